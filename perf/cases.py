@@ -399,10 +399,10 @@ def tolerance(case):
         return {"rel": 1e-13, "max": 1e-11} if case["dtype"] == "f64" else {"rel": 2e-6, "max": 1e-4}
     # Two correct solves stop within an iteration or two of each other at the same relative residual;
     # the error that leaves in x was measured against the exact solution: 1.3 (256^2 CG) and 0.5
-    # (128^3 CG) times the residual, 5 (64^3 BiCGStab), 0.6 (128^3 GMRES), 0.1 and less for the
-    # refined solves; it grows with the condition number, the square of the side.
+    # (128^3 CG) times the residual, 5 to 10 (64^3 BiCGStab), 1 (128^3 GMRES), 0.04 to 10
+    # (refined solves) over seeds; it grows with the condition number, the square of the side.
     side = 500 if kind == "serve" else max(case["nx"], case["ny"], case["nz"])
-    return {"rel": case["residue"] * max(20.0, 8e-5 * side * side)}
+    return {"rel": case["residue"] * max(50.0, 8e-5 * side * side)}
 
 
 def exact(case, seed):
