@@ -211,6 +211,57 @@ def test_ilu0_wide_levels_follow_the_oracle(tnl, dev, fmt):
     assert ok32 and its32 <= its + 5
 
 
+def _ilu_matrix(kind):
+    """Matrices whose triangular sweeps take each path of the device schedule."""
+    rng = np.random.default_rng(17)
+    if kind == "chain":  # every level one row, an odd number of them
+        n, per = 1501, [np.array([i - 1]) if i else np.array([], int) for i in range(1501)]
+    elif kind == "long rows":  # more entries than are fetched ahead, mixed lengths in a level
+        n = 4000
+        per = [np.unique(rng.integers(max(0, i - 900), max(i, 1), rng.integers(0, 12) if i % 7 else 40)) for i in range(n)]
+    elif kind == "far columns":  # dependencies older than the 16384 solution entries kept in LDS
+        n = 45000
+        per = [np.unique(np.concatenate([[i - 1500], rng.integers(0, i - 1500, 2)])) if i > 1500 else np.array([], int)
+               for i in range(n)]
+    else:  # "wide levels": levels on both sides of 4096 rows
+        sizes = [4096, 4097, 3, 1, 1025, 6000, 4095, 64]
+        start = np.concatenate([[0], np.cumsum(sizes)])
+        n, per = int(start[-1]), []
+        for lv, size in enumerate(sizes):
+            for k in range(size):
+                per.append(np.array([], int) if lv == 0 else np.unique(
+                    np.concatenate([rng.integers(start[lv - 1], start[lv], 1), rng.integers(0, start[lv], 2)])))
+    rows, cols, vals = [], [], []
+    for i in range(n):
+        low = per[i][per[i] < i]
+        up = [j for j in range(i + 1, min(n, i + 1 + i % 5))]
+        c = np.concatenate([low, [i] * (2 if i % 11 == 3 else 1), up]).astype(np.int32)
+        v = rng.uniform(-1, 1, len(c))
+        v[c == i] = 2.0 + len(c) / (2 if i % 11 == 3 else 1)
+        rows.append(len(c))
+        cols.append(c)
+        vals.append(v)
+    rp = np.concatenate([[0], np.cumsum(rows)]).astype(np.int32)
+    return rp, np.concatenate(cols), np.concatenate(vals)
+
+
+@pytest.mark.parametrize("kind", ["chain", "long rows", "far columns", "wide levels"])
+def test_ilu0_sweep_paths_follow_the_oracle(tnl, dev, kind):
+    """The triangular sweeps give TNL's bits on every path (rows longer than the fetched entries, a
+    second entry on the diagonal, columns older than the LDS ring, one-row and device-wide levels),
+    so the first residuals differ by the rounding of the solver's dot products only: sums of 45,000
+    terms in another order, about 1e-13 relative, a few of them per iteration."""
+    rp, c, v = _ilu_matrix(kind)
+    b = W.uniform_vector(len(rp) - 1, 5)
+    kw = dict(convergence_residue=1e-30, max_iterations=3, preconditioner=2)
+    ref = O.solve("bicgstab", rp, c, v, b, **kw)
+    _, _, _, hist, _ = _run_device_solver(tnl, dev, "bicgstab", rp, c, v, b, fmt="CSRScalar", **kw)
+    print(kind, hist[:4], ref["history"][:4], flush=True)
+    np.testing.assert_allclose(hist[:3], ref["history"][:3], rtol=1e-9)
+    _, _, _, h32, _ = _run_device_solver(tnl, dev, "bicgstab", rp, c, v, b, fmt="CSRScalar", dtype="f32", **kw)
+    np.testing.assert_allclose(h32[:2], ref["history"][:2], rtol=2e-3)  # FP32 factors and vectors
+
+
 def test_ilu0_refuses_rows_without_an_upper_entry(tnl, dev):
     # row 2 holds only a column below the diagonal: no U_22 to divide by
     rp = np.array([0, 1, 2, 3], np.int32)

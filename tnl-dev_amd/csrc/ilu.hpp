@@ -8,26 +8,37 @@ namespace tnlhip {
 
 struct Ilu0
 {
-   // one launch of a level schedule: a single level spread over the device, or a run of
-   // consecutive small levels processed by one workgroup with a barrier between levels
+   // one launch of a sweep: a single level spread over the device, or a run of consecutive small
+   // levels taken step by step by one workgroup
    struct Launch
    {
       int32_t firstLevel, lastLevel;  // [first, last)
+      int32_t firstStep, steps;
+      int32_t firstSlice, slices;
       bool wide;
    };
-   struct Schedule
+   // a triangular factor in level order
+   struct Sweep
    {
-      DeviceArray< int32_t > order;   // rows by level
-      std::vector< int32_t > levels;  // level boundaries into order (host copy)
+      DeviceArray< int32_t > order;     // row at each position
+      DeviceArray< int32_t > position;  // position of each row
+      std::vector< int32_t > levels;    // level boundaries in positions (host copy)
       DeviceArray< int32_t > levelsDevice;
       std::vector< Launch > launches;
+      DeviceArray< int32_t > len, steps, slices, sliceRest, slots, restCol;
+      DeviceArray< uint8_t > val, diag, restVal;
+      int32_t positions = 0, nslices = 0;
+      int32_t rest = 0;               // entries in the rest arrays
+      bool longRows = false;          // which W and D the sweep takes
    };
 
    int32_t n = 0;
    int dtype = TNLHIP_F64;  // value type of the factors and vectors (TNLHIP_F64 or TNLHIP_F32)
-   DeviceArray< int32_t > Lrp, Lc, Urp, Uc;
+   DeviceArray< int32_t > Lrp, Lc, Urp, Uc;  // the factors in row order, until the sweeps are packed
    DeviceArray< uint8_t > Lv, Uv;
-   Schedule lower, upper;
+   Sweep lower, upper;
+   DeviceArray< int32_t > between;  // lower position of the row at each upper position
+   DeviceArray< uint8_t > work;     // two vectors in level order
 
    // symbolic split and level schedules on the host, numeric factorization on the device
    void build( const Matrix& A, int vectorDtype, hipStream_t stream );
