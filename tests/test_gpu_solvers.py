@@ -187,6 +187,79 @@ def test_graph_replay_matches_direct_launches(tnl, dev, method, precond):
     np.testing.assert_array_equal(runs[0][3], runs[1][3])
 
 
+def _restart_blocks(m):
+    """m copies of a 3x3 system whose residual after one BiCGStab step is exactly orthogonal to r*,
+    so that the restart (BICGStab.hpp:88-95) is taken at once."""
+    block = np.array([[2.0, 1.0, -1.0], [1.0, 3.0, 1.0], [1.0, -1.0, 2.0]])
+    rp = np.arange(3 * m + 1, dtype=np.int32) * 3
+    cols = (np.repeat(np.arange(m), 9) * 3 + np.tile(np.tile([0, 1, 2], 3), m)).astype(np.int32)
+    return rp, cols, np.tile(block.ravel(), m), np.tile([1.0, 0.0, 0.0], m)
+
+
+@pytest.mark.parametrize("fmt", ["CSRScalar", "CSRAdaptive", "Ellpack", "SlicedEllpack", "ChunkedEllpack", "BiEllpack"])
+@pytest.mark.parametrize("n", [1, 2, 63, 257, 1025, 4097, 70001])
+def test_fused_iterations_follow_the_oracle(tnl, dev, fmt, n):
+    # tridiagonal, nonsymmetric for BiCGStab: sizes around wavefronts, workgroups, 16-byte lanes and
+    # partial counts; x at an odd 8-byte offset, so that the passes' narrow loads run
+    for method in ("cg", "bicgstab"):
+        up = -1.0 if method == "cg" else -0.7
+        i = np.arange(n)
+        r = np.concatenate([i[1:], i, i[:-1]])
+        c = np.concatenate([i[1:] - 1, i, i[:-1] + 1])
+        v = np.concatenate([np.full(n - 1, -1.0), 2.2 + 0.3 * np.cos(i), np.full(n - 1, up)])
+        o = np.lexsort((c, r))
+        rp = np.zeros(n + 1, np.int32)
+        np.cumsum(np.bincount(r, minlength=n), out=rp[1:])
+        cols, vals = c[o].astype(np.int32), v[o]
+        b = W.uniform_vector(n, 11)
+        for pre in (0, 1):
+            p = dict(convergence_residue=1e-10, max_iterations=60, preconditioner=pre)
+            ref = O.solve(method, rp, cols, vals, b, **p)
+            A = tnl.SparseMatrix.from_csr(rp, cols, vals, format=fmt, dtype="f64")
+            s = tnl.getLinearSolver(method)
+            s.setMatrix(A)
+            s.setup(**p)
+            bd, xd = t(b, dev), torch.zeros(n + 1, dtype=torch.float64, device=dev)[1:]
+            s.solve(bd, xd)
+            h = s.getResidualHistory()
+            # up to where the residual is rounding alone (one or two rows are solved in as many steps,
+            # and what is left may be 0, so the oracle's BiCGStab divides 0 by 0)
+            with np.errstate(invalid="ignore"):
+                m = min(12, int(np.argmin(np.append(ref["history"] > 1e-13, False))))
+            assert len(h) >= m >= 1
+            # the sums of up to 70001 products in another order: 1e-13 each, amplified by the steps
+            np.testing.assert_allclose(h[:m], ref["history"][:m], rtol=1e-8, atol=1e-14)
+            if n <= 2:
+                continue
+            assert abs(s.getIterations() - ref["iterations"]) <= 1
+            np.testing.assert_allclose(xd.cpu().numpy(), ref["x"], rtol=0, atol=1e-8 * np.abs(ref["x"]).max())
+
+
+@pytest.mark.parametrize("m", [1, 700, 110000])  # the last beyond the rows whose operand the product forms
+@pytest.mark.parametrize("use_graph", [0, 1])
+def test_bicgstab_restart_follows_the_oracle(tnl, dev, m, use_graph):
+    rp, cols, vals, b = _restart_blocks(m)
+    p = dict(convergence_residue=1e-12, max_iterations=40)
+    ref = O.solve("bicgstab", rp, cols, vals, b, **p)
+    ok, its, _, h, x = _run_device_solver(tnl, dev, "bicgstab", rp, cols, vals, b, fmt="SlicedEllpack",
+                                          use_graph=use_graph, **p)
+    k = min(len(h), len(ref["history"]), 4)  # the steps before the residual is at rounding level
+    np.testing.assert_allclose(h[:k], ref["history"][:k], rtol=1e-9, atol=1e-13)
+    assert abs(its - ref["iterations"]) <= 1 and ok == bool(ref["converged"])
+
+
+@pytest.mark.parametrize("method", ["cg", "bicgstab"])
+@pytest.mark.parametrize("most", [0, 1, 2, 11, 12, 13, 29])
+def test_iteration_limits_of_fused_solves(tnl, dev, method, most):
+    rp, c, v = W.laplacian_2d(24)
+    b = W.uniform_vector(len(rp) - 1, 5)
+    p = dict(convergence_residue=1e-30, max_iterations=most)
+    ref = O.solve(method, rp, c, v, b, **p)
+    ok, its, _, h, x = _run_device_solver(tnl, dev, method, rp, c, v, b, fmt="SlicedEllpack", **p)
+    assert not ok and its == ref["iterations"] and len(h) == len(ref["history"])
+    np.testing.assert_allclose(x, ref["x"], rtol=0, atol=1e-7 * np.abs(ref["x"]).max() + 1e-300)
+
+
 @pytest.mark.parametrize("fmt", ["SlicedEllpack", "CSRAdaptive"])
 def test_ilu0_wide_levels_follow_the_oracle(tnl, dev, fmt):
     """ILU(0) on the 64^3 Laplacian: the anti-diagonal planes hold up to 3072 rows, so the

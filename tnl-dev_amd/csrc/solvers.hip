@@ -15,6 +15,7 @@
 #include <memory>
 #include <type_traits>
 #include "ilu.hpp"
+#include "krylov.hpp"
 
 #include <cstdio>
 #include "matrix.hpp"
@@ -24,47 +25,6 @@
 #include <limits>
 
 namespace tnlhip {
-
-// ------------------------------------------------------------------ device state
-
-struct State
-{
-   double normb, residue, s1, s2, alpha, beta, omega, rho, rho_old, r_ast_sqnorm, normw, tmp, beta_gm;
-   double pad_;
-   int32_t it;
-   int32_t flags[ 2 ];  // [0] done (stop this solve / this GMRES cycle), [1] auxiliary gate
-   int32_t histLen;
-   int32_t o_steps;
-   int32_t breakdown;
-   int32_t stop;  // solve finished (GMRES: the outer loop must not continue)
-   int32_t pad2_;
-};
-
-struct Stop
-{
-   int32_t maxIt, minIt;
-   double conv, div;
-};
-
-// IterativeSolver::checkNextIteration (IterativeSolver.hpp:116-124)
-__device__ __forceinline__ bool checkNext( const State& s, const Stop& p )
-{
-   const double r = s.residue;
-   return ! ( isnan( r ) || s.it > p.maxIt || ( r > p.div && s.it >= p.minIt ) || ( r < p.conv && s.it >= p.minIt ) );
-}
-
-// IterativeSolver::setResidue with the residual history (IterativeSolver.hpp:189-200): each call
-// records (residue, the iteration count at that moment), the two fields of a history-file line
-__device__ __forceinline__ void setResidue( State& s, double r, double* hist, int64_t cap )
-{
-   s.residue = r;
-   if( s.histLen < cap ) {
-      hist[ 2 * (int64_t) s.histLen ] = r;
-      hist[ 2 * (int64_t) s.histLen + 1 ] = (double) s.it;
-   }
-   s.histLen++;
-}
-
 
 // ------------------------------------------------------------------ generic kernels
 
@@ -551,6 +511,71 @@ void runChunks( SolverImpl& S, Iter&& iteration )
    }
 }
 
+// The same for solves whose fused passes alternate between two sets of buffers: iteration( odd )
+// queues one iteration, `next` is the number of the next one and decides the set.  A solve that
+// stops with flags[1] set asks the host for `restart()` and goes on with the iteration that stopped.
+template< typename Iter, typename Restart >
+void runAlternating( SolverImpl& S, Iter&& iteration, Restart&& restart )
+{
+   constexpr int kGraphIters = 16;  // even: a replay leaves the sets as it found them
+   struct Graph
+   {
+      hipGraph_t g = nullptr;
+      hipGraphExec_t e = nullptr;
+      ~Graph()
+      {
+         if( e )
+            (void) hipGraphExecDestroy( e );
+         if( g )
+            (void) hipGraphDestroy( g );
+      }
+   } graph;
+   int64_t next = 0;
+   // the iteration after the last one allowed only checks the stopping rule
+   const int64_t limit = (int64_t) S.params.max_iterations + 3;
+   int reps = 1, chunk = 16;
+   while( true ) {
+      if( next < 12 || next % 2 != 0 || ! S.params.use_graph ) {
+         int64_t end = next < 4 ? 4 : 12;
+         if( next >= 12 ) {
+            end = S.params.use_graph ? next + 1 : next + chunk;
+            chunk = std::min( chunk * 2, 64 );
+         }
+         for( ; next < end && next < limit; next++ )
+            iteration( next % 2 != 0 );
+      }
+      else {
+         if( ! graph.e ) {
+            TNLHIP_CHECK( hipStreamBeginCapture( S.stream, hipStreamCaptureModeThreadLocal ) );
+            try {
+               for( int k = 0; k < kGraphIters; k++ )
+                  iteration( k % 2 != 0 );
+            }
+            catch( ... ) {
+               hipGraph_t broken = nullptr;
+               (void) hipStreamEndCapture( S.stream, &broken );
+               if( broken )
+                  (void) hipGraphDestroy( broken );
+               throw;
+            }
+            TNLHIP_CHECK( hipStreamEndCapture( S.stream, &graph.g ) );
+            TNLHIP_CHECK( hipGraphInstantiate( &graph.e, graph.g, nullptr, nullptr, 0 ) );
+         }
+         for( int r = 0; r < reps && next < limit; r++, next += kGraphIters )
+            TNLHIP_CHECK( hipGraphLaunch( graph.e, S.stream ) );
+         reps = std::min( reps * 2, 4 );
+      }
+      const State h = readState( S );
+      if( h.flags[ 0 ] && h.flags[ 1 ] ) {
+         restart();
+         next = h.it;
+         continue;
+      }
+      if( h.flags[ 0 ] || next >= limit )
+         return;
+   }
+}
+
 // ================================================================== CG
 
 template< typename T >
@@ -668,31 +693,6 @@ struct CgDirectionOp
    __device__ void load() { beta = st->beta; }
    __device__ void operator()( int64_t i ) const { p[ i ] = (T) ( (double) zr[ i ] + beta * (double) p[ i ] ); }
 };
-
-// The sum a reduction's final kernel would form, formed instead by every workgroup of the next
-// kernel from the same partials in the same order (sumPartials), so each workgroup holds the
-// same bits; the next kernel's workgroup 0 then does the final kernel's state update.  It saves
-// the final kernel's launch; no workgroup may read a state field that workgroup 0 of the same
-// launch writes.
-__device__ __forceinline__ double foldPartials1( ReduceSlot slot, int grid )
-{
-   __shared__ double tot[ 1 ];
-   sumPartials< 1 >( slot, grid, tot );
-   return tot[ 0 ];
-}
-
-__device__ __forceinline__ void foldPartials2( ReduceSlot slot, int grid, double ( &v )[ 2 ] )
-{
-   __shared__ double tot[ 2 ];
-   sumPartials< 2 >( slot, grid, tot );
-   v[ 0 ] = tot[ 0 ];
-   v[ 1 ] = tot[ 1 ];
-}
-
-__device__ __forceinline__ bool leadLane()
-{
-   return blockIdx.x == 0 && threadIdx.x == 0;
-}
 
 template< typename T >
 struct CgUpdateFoldOp
@@ -842,6 +842,69 @@ void solveCGSeparate( SolverImpl& S, const void* b, void* xv )
 }
 
 template< typename T >
+struct CgFusedInitOp : NoScalars
+{
+   // z = r / diag (when preconditioned); p = 0 (the first direction has beta = 0); acc += r * (z or r)
+   T* p;
+   T* z;
+   const T* r;
+   const T* diag;
+   __device__ void operator()( int64_t i, double ( &acc )[ 1 ] ) const
+   {
+      const T ri = r[ i ];
+      T zi = ri;
+      if( diag ) {
+         zi = ri / diag[ i ];
+         z[ i ] = zi;
+      }
+      p[ i ] = 0;
+      acc[ 0 ] += (double) ri * (double) zi;
+   }
+};
+
+// CG over the fused products: an iteration first closes the one before it (the residue, the
+// stopping rule, beta) and then takes its step.  Two launches where the direction is formed in the
+// product, three where it has a pass of its own.
+template< typename T >
+void solveCGFused( SolverImpl& S, const void* b, T* x, int dotGrid )
+{
+   T* r = (T*) S.vec( 0 );
+   T* p[ 2 ] = { (T*) S.vec( 1 ), (T*) S.vec( 4 ) };
+   T* Ap = (T*) S.vec( 2 );
+   T* z = (T*) S.vec( 3 );
+   const T* diag = S.params.preconditioner == 1 ? (const T*) S.diag.ptr : nullptr;
+   const T* zr = diag ? z : r;
+   const Gate always{ nullptr, 0 }, running{ S.state.ptr->flags, 1 };
+   const Stop stop = S.stopRule();
+   State* st = S.state.ptr;
+   const ReduceSlot dot = S.ws.slot( 1 ), upd = S.ws.slot( 2 );
+   const int grid = passGrid< T >( S.n );
+   const bool fuse = fuseOperand( *S.A );
+   const CgNext next{ st, S.hist.ptr, S.histCap, stop, { upd, grid } };
+   const CgAlpha alpha{ st, S.hist.ptr, S.histCap, { dot, dotGrid } };
+   computeNormb< T >( S, b, z );
+   residual< T >( S, b, x, r, always, false );  // CG.hpp:40-41: r = b - A x
+   fusedReduceKernel< 1 ><<< grid, kReduceBlock, 0, S.stream >>>( S.n, CgFusedInitOp< T >{ {}, p[ 0 ], z, r, diag }, upd,
+                                                                  always );
+   runAlternating(
+      S,
+      [ & ]( bool odd ) {
+         T* pNew = fuse ? p[ odd ? 0 : 1 ] : p[ 0 ];
+         if( fuse )
+            fusedProduct( *S.A, CgDirectionOperand< T >{ zr, p[ odd ? 1 : 0 ], pNew, next }, (const T*) nullptr,
+                          (const T*) nullptr, Ap, dot, running, S.stream );
+         else {
+            launchPass< 0, T >( S.n, CgDirectionPass< T >{ pNew, zr, next }, upd, running, S.stream );
+            fusedProduct( *S.A, DotOperand< T >{ {}, pNew }, (const T*) pNew, (const T*) nullptr, Ap, dot, running,
+                          S.stream );
+         }
+         launchPass< 1, T >( S.n, CgUpdatePass< T >{ x, r, z, pNew, Ap, diag, aligned16( x ), alpha }, upd, running,
+                             S.stream );
+      },
+      [] {} );
+}
+
+template< typename T >
 void solveCG( SolverImpl& S, const void* b, void* xv )
 {
    if( S.params.preconditioner >= 2 ) {
@@ -857,6 +920,10 @@ void solveCG( SolverImpl& S, const void* b, void* xv )
    const T* diag = S.params.preconditioner == 1 ? (const T*) S.diag.ptr : nullptr;
    const Gate always{ nullptr, 0 }, running{ S.state.ptr->flags, 1 };
    const Stop stop = S.stopRule();
+   if( const int grid = fusedGrid( *S.A ) ) {
+      solveCGFused< T >( S, b, x, grid );
+      return;
+   }
    computeNormb< T >( S, b, z );
    residual< T >( S, b, x, r, always, false );  // CG.hpp:40-41: r = b - A x
    launchReduce< 1 >( S.n, CgInitOp< T >{ {}, p, z, r, diag }, FinCgInit{ S.state.ptr, S.hist.ptr, S.histCap, stop },
@@ -1140,6 +1207,107 @@ struct FinPromoteStop
 };
 
 template< typename T >
+struct BiFusedInitOp : NoScalars
+{
+   // r_ast = r; p = Ap = 0 (the first direction has beta = 0); acc = { (r, r_ast), (r, r) }
+   T* p;
+   T* Ap;
+   T* rast;
+   const T* r;
+   __device__ void operator()( int64_t i, double ( &acc )[ 2 ] ) const
+   {
+      const T ri = r[ i ];
+      p[ i ] = 0;
+      Ap[ i ] = 0;
+      rast[ i ] = ri;
+      acc[ 0 ] += (double) ri * (double) ri;
+      acc[ 1 ] += (double) ri * (double) ri;
+   }
+};
+
+template< typename T >
+struct BiFusedRestartOp : NoScalars
+{
+   // r_ast = r; acc = { (r, r_ast), (r, r) }
+   T* rast;
+   const T* r;
+   __device__ void operator()( int64_t i, double ( &acc )[ 2 ] ) const
+   {
+      const T ri = r[ i ];
+      rast[ i ] = ri;
+      acc[ 0 ] += (double) ri * (double) ri;
+      acc[ 1 ] += (double) ri * (double) ri;
+   }
+};
+
+// the solve goes on after a restart (FinBiRestart's part that the next direction does not do)
+struct FinBiResume
+{
+   State* st;
+   __device__ void operator()() const
+   {
+      st->flags[ 0 ] = st->flags[ 1 ] = 0;
+      st->started = 2;
+   }
+};
+
+// BiCGStab over the fused products: an iteration first closes the one before it (rho, the restart
+// test, the residue, the stopping rule, beta), then takes its two half steps.  Three launches
+// where the operands are formed in the products, five where they have passes of their own.  The
+// rare restart is the host's: the queued launches stop, and the solve resumes at that iteration.
+template< typename T >
+void solveBiCGStabFused( SolverImpl& S, const void* b, T* x, int dotGrid )
+{
+   T* r = (T*) S.vec( 0 );
+   T* rast = (T*) S.vec( 1 );
+   T* p[ 2 ] = { (T*) S.vec( 2 ), (T*) S.vec( 6 ) };
+   T* s = (T*) S.vec( 3 );
+   T* Ap[ 2 ] = { (T*) S.vec( 4 ), (T*) S.vec( 7 ) };
+   T* As = (T*) S.vec( 5 );
+   const T* diag = S.params.preconditioner == 1 ? (const T*) S.diag.ptr : nullptr;
+   const Gate always{ nullptr, 0 }, running{ S.state.ptr->flags, 1 };
+   const double eps = std::numeric_limits< T >::epsilon();
+   State* st = S.state.ptr;
+   const int grid = passGrid< T >( S.n );
+   const ReduceSlot dot = S.ws.slot( 0 ), om = S.ws.slot( 1 ), upd = S.ws.slot( 2 );
+   const BiNext next{ st, S.hist.ptr, S.histCap, S.stopRule(), eps * eps, { upd, grid } };
+   const BiAlpha alpha{ st, { dot, dotGrid } };
+   const BiOmega omega{ st, { om, dotGrid } };
+   const bool fuse = fuseOperand( *S.A );
+   computeNormb< T >( S, b, p[ 1 ] );
+   residual< T >( S, b, x, r, always );
+   fusedReduceKernel< 2 ><<< grid, kReduceBlock, 0, S.stream >>>(
+      S.n, BiFusedInitOp< T >{ {}, p[ 0 ], Ap[ 0 ], rast, r }, upd, always );
+   runAlternating(
+      S,
+      [ & ]( bool odd ) {
+         T* pNew = fuse ? p[ odd ? 0 : 1 ] : p[ 0 ];
+         T* ApNew = fuse ? Ap[ odd ? 0 : 1 ] : Ap[ 0 ];
+         if( fuse ) {
+            fusedProduct( *S.A, BiDirectionOperand< T >{ r, p[ odd ? 1 : 0 ], Ap[ odd ? 1 : 0 ], pNew, rast, next },
+                          (const T*) nullptr, diag, ApNew, dot, running, S.stream );
+            fusedProduct( *S.A, BiSOperand< T >{ r, ApNew, s, alpha }, (const T*) nullptr, diag, As, om, running,
+                          S.stream );
+         }
+         else {
+            launchPass< 0, T >( S.n, BiDirectionPass< T >{ pNew, r, ApNew, next }, upd, running, S.stream );
+            fusedProduct( *S.A, DotOperand< T >{ {}, rast }, (const T*) pNew, diag, ApNew, dot, running, S.stream );
+            launchPass< 0, T >( S.n, BiSPass< T >{ s, r, ApNew, alpha }, om, running, S.stream );
+            fusedProduct( *S.A, DotSquareOperand< T >{ {}, s }, (const T*) s, diag, As, om, running, S.stream );
+         }
+         launchPass< 2, T >( S.n, BiUpdatePass< T >{ x, r, pNew, s, As, rast, aligned16( x ), omega }, upd, running,
+                             S.stream );
+      },
+      [ & ] {
+         // r = M^{-1}(b - A x); r_ast = r; rho = r_ast_sqnorm = (r, r) (BICGStab.hpp:88-95)
+         residual< T >( S, b, x, r, always );
+         fusedReduceKernel< 2 ><<< grid, kReduceBlock, 0, S.stream >>>( S.n, BiFusedRestartOp< T >{ {}, rast, r }, upd,
+                                                                        always );
+         launchScalar( FinBiResume{ st }, always, S.stream );
+      } );
+}
+
+template< typename T >
 void solveBiCGStab( SolverImpl& S, const void* b, void* xv )
 {
    // vectors: r, r_ast, p, s, Ap, As, M_tmp
@@ -1155,6 +1323,11 @@ void solveBiCGStab( SolverImpl& S, const void* b, void* xv )
    const Gate always{ nullptr, 0 }, running{ S.state.ptr->flags, 1 }, restart{ S.state.ptr->flags, 2 };
    const Stop stop = S.stopRule();
    const double eps = std::numeric_limits< T >::epsilon();
+   const int fused = ! exact && S.params.preconditioner <= 1 ? fusedGrid( *S.A ) : 0;
+   if( fused ) {
+      solveBiCGStabFused< T >( S, b, x, fused );
+      return;
+   }
    computeNormb< T >( S, b, Mt );
    residual< T >( S, b, x, r, always );
    launchReduce< 1 >( S.n, OpCopy2< T >{ {}, p, rast, s, r }, FinRhoInit{ S.state.ptr, S.hist.ptr, S.histCap, stop },
@@ -2629,9 +2802,9 @@ void prepare( SolverImpl& S )
    // column stride aligned to 256 bytes, as GMRES::setSize does for GPUs (GMRES.hpp:765-773)
    const int64_t per = 256 / (int64_t) S.vbytes;
    S.ld = ( S.n + per - 1 ) / per * per;
-   int nvec = 4;
+   int nvec = 5;
    if( S.method == TNLHIP_BICGSTAB )
-      nvec = 7;
+      nvec = 8;
    if( S.method == TNLHIP_TFQMR )
       nvec = 8;
    if( S.method == TNLHIP_BICGSTABL ) {

@@ -15,6 +15,7 @@ namespace tnlhip {
 template< typename A, typename Y >
 struct Keeper
 {
+   static constexpr bool kPlain = true;
    Y* y;
    A alpha, beta;
    const Y* diag;
@@ -26,6 +27,11 @@ struct Keeper
    bool streamY = true;
    const Y* rhs = nullptr;   // mode 5
    const Y* prev = nullptr;  // mode 5
+   // the row kernels' other calls (spmv_kernels.hpp): a plain product has nothing to do there
+   __device__ __forceinline__ void prefetch() {}
+   __device__ __forceinline__ bool begin() { return true; }
+   __device__ __forceinline__ Y at( const Y* x, int64_t c ) const { return x[ c ]; }
+   __device__ __forceinline__ void finish() {}
    __device__ __forceinline__ bool closed() const
    {
       if( gateMode == 0 )
