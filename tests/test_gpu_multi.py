@@ -138,3 +138,43 @@ def test_block_product_unaligned_blocks_take_the_scalar_lanes(tnl, dev):
     torch.cuda.synchronize()
     assert np.array_equal(Yu.cpu().numpy(), want)
     assert np.array_equal(Ya.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("fmt", ["CSRScalar", "Ellpack", "SlicedEllpack", "ChunkedEllpack"])
+@pytest.mark.parametrize("dt", ["f64", "f32"])
+@pytest.mark.parametrize("k", [3, 5, 7, 9, 12, 16, 17, 33, 64])
+def test_short_rows_equal_the_columns_one_by_one(tnl, dev, fmt, dt, k):
+    # 65 x 67 x 61 rows: ragged tiles, enough of them for the walk of 8 at k >= 12; a few rows beyond 8
+    # slots in the CSR forms; X and Y at odd element offsets; a row range that starts inside a tile; the
+    # one-vector product of SlicedEllpack sums every row in the same order with the same rounding
+    rng = np.random.default_rng(k)
+    for box, longs in (((65, 67, 61), fmt == "CSRScalar"), ((9, 5, 3), True)):
+        rp, c, v = W._stencil(box[::-1], [(d, 1.0) for d in ((-1, 0, 0), (0, -1, 0), (0, 0, -1), (0, 0, 0), (0, 0, 1),
+                                                            (0, 1, 0), (1, 0, 0))])
+        n = len(rp) - 1
+        rows = np.repeat(np.arange(n), np.diff(rp))
+        key = rows.astype(np.int64) * n + c
+        if longs:
+            extra = rng.choice(n, 5, replace=False)
+            key = np.unique(np.concatenate([key] + [r * n + rng.choice(n, 40) for r in extra.astype(np.int64)]))
+        rows, c = key // n, (key % n).astype(np.int32)
+        rp = np.zeros(n + 1, np.int32)
+        np.cumsum(np.bincount(rows, minlength=n), out=rp[1:])
+        v = rng.uniform(-1, 1, len(c))
+        td = torch.float64 if dt == "f64" else torch.float32
+        A = tnl.SparseMatrix.from_csr(rp, c, v, format=fmt, dtype=dt)
+        B = tnl.SparseMatrix.from_csr(rp, c, v, format="CSRScalar", dtype=dt)
+        X = torch.tensor(rng.uniform(-1, 1, n * k + 1), dtype=td, device=dev)[1:].view(n, k)
+        Y0 = torch.tensor(rng.uniform(-1, 1, n * k + 1), dtype=td, device=dev)[1:].view(n, k)
+        want = torch.stack([B.vectorProduct(X[:, j].contiguous(), torch.zeros(n, dtype=td, device=dev))
+                            for j in range(k)], 1)
+        Y = Y0.clone()
+        A.vectorProductMulti(X, Y)
+        assert torch.equal(Y, want), (box, "y = A x")
+        for alpha, beta, lo, hi in ((-1.0, 1.0, 0, n), (0.5, -2.0, 7, n - 3)):
+            Y = torch.empty(n * k + 1, dtype=td, device=dev)[1:].view(n, k).copy_(Y0)
+            A.vectorProductMulti(X, Y, alpha, beta, lo, hi)
+            ref = Y0.double() * beta + alpha * want.double()
+            eps = 2.0 ** (-50 if dt == "f64" else -21)
+            assert (Y[lo:hi].double() - ref[lo:hi]).abs().max() <= eps * 8
+            assert torch.equal(Y[:lo], Y0[:lo]) and torch.equal(Y[hi:], Y0[hi:])

@@ -35,12 +35,14 @@ __global__ void fillPaddingKernel( int64_t n, int32_t* cols, V* vals )
 }
 
 // One lane per row, sequential over the row: local indexes must be assigned in source order.
+// info[0]: a row's capacity was exceeded; info[1]: the largest |column - row| stored.
 template< typename View, typename V >
 __global__ void scatterFromCsrKernel( int32_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ scol,
                                       const double* __restrict__ sval, View dst, int32_t* __restrict__ dcol,
-                                      V* __restrict__ dval, int32_t* __restrict__ overflow, int keepZeros )
+                                      V* __restrict__ dval, int32_t* __restrict__ info, int keepZeros )
 {
    const int64_t stride = (int64_t) gridDim.x * blockDim.x;
+   int32_t reach = 0;
    for( int64_t r = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; r < n; r += stride ) {
       int32_t local = 0;
       const int32_t cap = dst.size( (int32_t) r );
@@ -49,16 +51,21 @@ __global__ void scatterFromCsrKernel( int32_t n, const int32_t* __restrict__ rp,
          const int32_t c = scol[ k ];
          if( ( keepZeros || v != 0.0 ) && c != -1 ) {
             if( local >= cap ) {
-               *overflow = 1;
+               info[ 0 ] = 1;
                break;
             }
             const int64_t g = dst.global( (int32_t) r, local++ );
             dcol[ g ] = c;
             if( dval )
                dval[ g ] = fromDouble< V >( v );
+            reach = max( reach, (int32_t) llabs( (int64_t) c - r ) );
          }
       }
    }
+   for( int o = kWave / 2; o > 0; o /= 2 )
+      reach = max( reach, __shfl_xor( reach, o, kWave ) );
+   if( threadIdx.x % kWave == 0 && reach > 0 )
+      atomicMax( info + 1, reach );
 }
 
 // Source row r, local order -> compressed CSR row (values as double) of capacity size(r).
@@ -120,8 +127,8 @@ __global__ void diagonalKernel( int32_t n, View v, const int32_t* __restrict__ c
 void convertFromCsrDevice( Matrix& A, const int32_t* rowPtr, const int32_t* cols, const double* vals,
                            hipStream_t stream, bool keepZeros )
 {
-   DeviceArray< int32_t > overflow( 1 );
-   TNLHIP_CHECK( hipMemsetAsync( overflow.ptr, 0, sizeof( int32_t ), stream ) );
+   DeviceArray< int32_t > info( 2 );
+   TNLHIP_CHECK( hipMemsetAsync( info.ptr, 0, 2 * sizeof( int32_t ), stream ) );
    withValueType( A.dtype, [ & ]( auto* tag ) {
       using V = std::remove_pointer_t< decltype( tag ) >;
       V* dval = reinterpret_cast< V* >( A.values.ptr );
@@ -131,14 +138,15 @@ void convertFromCsrDevice( Matrix& A, const int32_t* rowPtr, const int32_t* cols
       if( A.rows > 0 )
          withView( A, [ & ]( auto view ) {
             scatterFromCsrKernel<<< gridFor( A.rows, 256 ), 256, 0, stream >>>(
-               A.rows, rowPtr, cols, vals, view, A.columns.ptr, dval, overflow.ptr, keepZeros ? 1 : 0 );
+               A.rows, rowPtr, cols, vals, view, A.columns.ptr, dval, info.ptr, keepZeros ? 1 : 0 );
          } );
    } );
    TNLHIP_CHECK( hipGetLastError() );
-   int32_t ov = 0;
-   TNLHIP_CHECK( hipMemcpyAsync( &ov, overflow.ptr, sizeof( int32_t ), hipMemcpyDeviceToHost, stream ) );
+   int32_t got[ 2 ] = { 0, 0 };
+   TNLHIP_CHECK( hipMemcpyAsync( got, info.ptr, 2 * sizeof( int32_t ), hipMemcpyDeviceToHost, stream ) );
    TNLHIP_CHECK( hipStreamSynchronize( stream ) );
-   if( ov )
+   A.reach = got[ 1 ];
+   if( got[ 0 ] )
       throw Error( TNLHIP_ERROR_CAPACITY, "row capacity exceeded during conversion" );
 }
 

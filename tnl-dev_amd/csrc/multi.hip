@@ -11,14 +11,40 @@
 // over the row's slots, rounding each product (TNL's Host order: CSRScalarKernel.hpp:70-107 and
 // the padded formats' per-segment loops), so column j of Y equals TNL's product of column j of X
 // bit for bit; padding slots (column -1) are skipped.  Keepers as SparseMatrixView.hpp:447-471.
+#include "rowdist.hpp"
 #include "spmv.hpp"
+
+#include <algorithm>
+#include <type_traits>
 
 namespace tnlhip {
 
 namespace {
 
 constexpr int kMultiChunk = 8;  // slots of a row whose loads are in flight together
-constexpr int kMultiXcds = 8;   // workgroups are dispatched round-robin over the 8 XCDs
+constexpr int64_t kMultiManyTiles = 100000;  // tiles from which a wave of the short-row kernel walks 8 of them
+
+// Row blocks an XCD takes in a row before the next XCD's share begins.  A block gathers the X rows
+// within the matrix's reach of it; where an XCD sweeps a contiguous eighth of the rows, two reaches of X
+// rows pass through its L2 before one is read again.  A share of an eighth of the reach puts rows r - reach,
+// r and r + reach on the same XCD with an eighth of that in between.  128^3 Laplacian, k = 16 in
+// FP64 (reach 16384 rows, 2 MB of X): 239 us contiguous, 227 us in shares; where the window fits anyway
+// (3 reaches within a MiB) and where the reach is that of the matrix, contiguous eighths stay.
+int64_t multiChunk( const Matrix& M, int64_t blocks, int64_t rowsPerBlock, int64_t rowBytes )
+{
+   const int64_t whole = std::max< int64_t >( 1, ( blocks + kXcds - 1 ) / kXcds );
+   // (ChunkedEllpack's and BiEllpack's kernels are bound by their index maps: 328 us contiguous against 342)
+   const int kind = kindOf( M.format );
+   if( kind == KIND_CHUNKED || kind == KIND_BIELLPACK || M.reach <= 0 || 3 * M.reach * rowBytes <= ( 1 << 20 ) )
+      return whole;
+   return std::min( whole, std::max< int64_t >( 1, ( M.reach / kXcds + rowsPerBlock - 1 ) / rowsPerBlock ) );
+}
+
+__device__ __forceinline__ int64_t multiBlock( int32_t chunk )
+{
+   const int64_t xcd = blockIdx.x % kXcds, pos = blockIdx.x / kXcds;
+   return ( pos / chunk * kXcds + xcd ) * chunk + pos % chunk;
+}
 
 // VW-wide vector of the compute type (VW = 1: the scalar itself)
 template< typename A, int VW >
@@ -51,15 +77,14 @@ __global__ __launch_bounds__( 256 ) void multiProductKernel( View view, const in
                                                              const V* __restrict__ val, int32_t k,
                                                              const Y* __restrict__ X, Y* __restrict__ Yout, A alpha,
                                                              A beta, int mode, int32_t first, int32_t last,
-                                                             int32_t ncols )
+                                                             int32_t ncols, int32_t chunk )
 {
    constexpr int L = KP / VW;
    constexpr int kRowsPerBlock = 256 / L;
    using VA = typename Lanes< A, VW >::type;
    using VY = typename Lanes< Y, VW >::type;
    const int jq = threadIdx.x % L;
-   const int64_t block = (int64_t) ( blockIdx.x % kMultiXcds ) * ( gridDim.x / kMultiXcds ) + blockIdx.x / kMultiXcds;
-   const int64_t r = first + block * kRowsPerBlock + threadIdx.x / L;
+   const int64_t r = first + multiBlock( chunk ) * kRowsPerBlock + threadIdx.x / L;
    if( r >= last )
       return;
    // no columns: every slot is padding and X may be empty
@@ -135,14 +160,291 @@ void launchMultiW( const Matrix& M, int32_t k, const Y* X, Y* Yv, double alpha, 
    constexpr int kRowsPerBlock = 256 / ( KP / VW );
    const int64_t rows = last - first;
    int64_t blocks = ( rows + kRowsPerBlock - 1 ) / kRowsPerBlock;
-   blocks = ( blocks + kMultiXcds - 1 ) / kMultiXcds * kMultiXcds;
+   const int64_t chunk = multiChunk( M, blocks, kRowsPerBlock, (int64_t) k * sizeof( Y ) );
+   blocks = ( blocks + kXcds * chunk - 1 ) / ( kXcds * chunk ) * ( kXcds * chunk );
    TNLHIP_REQUIRE( blocks < ( 1ll << 31 ), "too many rows for one launch" );
    withView( M, [ & ]( auto view ) {
       multiProductKernel< KP, VW, V, A, Y ><<< (unsigned) blocks, 256, 0, st >>>(
          view, M.columns.ptr, reinterpret_cast< const V* >( M.values.ptr ), k, X, Yv, (A) alpha, (A) beta, mode, first,
-         last, M.cols );
+         last, M.cols, (int32_t) chunk );
    } );
    TNLHIP_CHECK( hipGetLastError() );
+}
+
+// ------------------------------------------------------------------ short rows
+
+// The words a lane loads to address the slots of one row, for the formats whose rows are one run of
+// equal steps (CSR, Ellpack, SlicedEllpack).  They are kept as loaded and combined where they are used:
+// arithmetic on them at the load would wait for it, and with it for every load under way.
+struct RowRun
+{
+   int32_t a = 0, b = 0;
+};
+__device__ __forceinline__ RowRun rowRun( const CsrView& v, int32_t r )
+{
+   return RowRun{ v.offsets[ r ], v.offsets[ r + 1 ] };
+}
+__device__ __forceinline__ RowRun rowRun( const EllpackView& v, int32_t ) { return RowRun{ 0, v.segmentSize }; }
+__device__ __forceinline__ RowRun rowRun( const SlicedView& v, int32_t r )
+{
+   return RowRun{ v.sliceOffsets[ r >> v.logSlice ], v.sliceSizes[ r >> v.logSlice ] };
+}
+__device__ __forceinline__ int32_t runSize( const CsrView&, RowRun m ) { return m.b - m.a; }
+__device__ __forceinline__ int32_t runSize( const EllpackView&, RowRun m ) { return m.b; }
+__device__ __forceinline__ int32_t runSize( const SlicedView&, RowRun m ) { return m.b; }
+__device__ __forceinline__ int64_t runStart( const CsrView&, RowRun m, int64_t ) { return m.a; }
+__device__ __forceinline__ int64_t runStart( const EllpackView&, RowRun, int64_t r ) { return r; }
+__device__ __forceinline__ int64_t runStart( const SlicedView& v, RowRun m, int64_t r )
+{
+   return m.a + ( r & ( ( 1 << v.logSlice ) - 1 ) );
+}
+__device__ __forceinline__ int64_t runStep( const CsrView& ) { return 1; }
+__device__ __forceinline__ int64_t runStep( const EllpackView& v ) { return v.alignedSize; }
+__device__ __forceinline__ int64_t runStep( const SlicedView& v ) { return (int64_t) 1 << v.logSlice; }
+
+template< typename View >
+constexpr bool kRunView = std::is_same_v< View, CsrView > || std::is_same_v< View, EllpackView > ||
+                          std::is_same_v< View, SlicedView >;
+
+// VW adjacent entries wherever they start (global loads need only element alignment)
+template< typename Y, int VW >
+struct Packed
+{
+   typedef Y type __attribute__( ( ext_vector_type( VW ), aligned( sizeof( Y ) ) ) );
+};
+
+// The product for rows of up to kMultiChunk slots (longer ones take the rest of their slots in a loop
+// of their own).  Bound by latency before it is bound by bytes: in multiProductKernel a wave lives
+// for one row per L lanes, through three dependent trips to memory (row, slots, X).  Here a
+// wave walks `tiles` tiles of 64 / L rows with the next tile's slots and the one after's row
+// loaded ahead, and X of the next tile under way while it sums this one.  A tile's slots are
+// loaded once, one lane each, and shared through wave-local LDS; the L lanes of a row read them
+// there.  Lane jq of a row takes columns j0 .. j0 + VW - 1, j0 = VW jq; when VW does not divide k the last
+// lane starts early enough to end at column k - 1 and stores only its own columns.  Every column is
+// summed left to right in the Host order, as in multiProductKernel.
+// 128^3 Laplacian, SlicedEllpack FP64, k = 16: 239 -> 209 us
+template< int L, int VW, typename V, typename A, typename Y, typename View >
+__global__ __launch_bounds__( 256 ) void multiShortKernel( View view, const int32_t* __restrict__ col,
+                                                           const V* __restrict__ val, int32_t k,
+                                                           const Y* __restrict__ X, Y* __restrict__ Yout, A alpha,
+                                                           A beta, int mode, int32_t first, int32_t last,
+                                                           int32_t ncols, int32_t chunk, int32_t tiles )
+{
+   constexpr int RW = kWave / L;  // rows of a tile
+   constexpr int S = kMultiChunk;
+   constexpr int PL = L >= S ? 1 : S / L;  // slots a lane loads
+   constexpr int kWaves = 256 / kWave;
+   using VY = typename Packed< Y, VW >::type;
+   __shared__ __align__( 16 ) int32_t sc[ kWaves ][ 2 ][ RW * S ];
+   __shared__ __align__( 16 ) A sv[ kWaves ][ 2 ][ RW * S ];
+   __shared__ int32_t sn[ kWaves ][ 2 ][ RW ];
+   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+   const int loadRow = lane % RW, loadSlot = lane / RW;  // as a loader: slots loadSlot, loadSlot + L, ...
+   const int myRow = lane / L, jq = lane % L;            // as a summer
+   const bool mine = VW * jq < k;
+   const int j0 = mine ? min( VW * jq, k - VW ) : 0;
+   const int64_t step = runStep( view );
+   // a workgroup takes `tiles` consecutive blocks of kWaves tiles, in the order of multiBlock
+   int64_t block = multiBlock( chunk ) * tiles;
+   auto nextBase = [ & ] {  // first row of the wave's next tile (past the last one: no rows)
+      const int64_t base = first + ( block * kWaves + wave ) * RW;
+      block++;
+      return base;
+   };
+   auto loadRun = [ & ]( int64_t base ) {
+      const int64_t r = base + loadRow;
+      RowRun m;
+      if( r < last )
+         m = rowRun( view, (int32_t) r );
+      return m;
+   };
+   struct Slots
+   {
+      int32_t c[ PL ];
+      V v[ PL ];
+      int32_t size;
+   };
+   auto loadSlots = [ & ]( RowRun m, int64_t base ) {
+      Slots s;
+      s.size = base + loadRow < last ? runSize( view, m ) : 0;
+      const int64_t start = runStart( view, m, base + loadRow );
+#pragma unroll
+      for( int j = 0; j < PL; j++ ) {
+         const int l = loadSlot + j * L;
+         s.c[ j ] = -1;
+         s.v[ j ] = V( 0.0f );
+         if( l < S && l < s.size ) {
+            const int64_t g = start + step * l;
+            s.c[ j ] = __builtin_nontemporal_load( col + g );
+            s.v[ j ] = val[ g ];
+         }
+      }
+      return s;
+   };
+   auto share = [ & ]( int buf, const Slots& s ) {
+      waveSync();
+#pragma unroll
+      for( int j = 0; j < PL; j++ ) {
+         const int l = loadSlot + j * L;
+         if( l < S ) {
+            sc[ wave ][ buf ][ loadRow * S + l ] = s.c[ j ];
+            sv[ wave ][ buf ][ loadRow * S + l ] = toCompute( s.v[ j ], A() );
+         }
+      }
+      if( loadSlot == 0 )
+         sn[ wave ][ buf ][ loadRow ] = s.size;
+      waveSync();
+   };
+   struct Gathered
+   {
+      VY x[ S ];
+      VY y;
+   };
+   const Y* xs = X + j0;
+   auto gather = [ & ]( int buf, int64_t base, Gathered& g ) {
+      const int64_t r = min( base + myRow, (int64_t) last - 1 );
+      const int32_t spare = (int32_t) min( r, (int64_t) ncols - 1 );  // padding reads a row that is read anyway
+#pragma unroll
+      for( int u = 0; u < S; u++ ) {
+         const int32_t c = sc[ wave ][ buf ][ myRow * S + u ];
+         g.x[ u ] = *reinterpret_cast< const VY* >( xs + (int64_t) ( c >= 0 ? c : spare ) * k );
+      }
+      if( mode >= 2 )
+         g.y = *reinterpret_cast< const VY* >( Yout + r * k + j0 );
+   };
+   auto finish = [ & ]( int buf, int64_t base, const Gathered& g ) {
+      const int64_t r = base + myRow;
+      A sum[ VW ] = {};
+#pragma unroll
+      for( int u = 0; u < S; u++ ) {
+         const int32_t c = sc[ wave ][ buf ][ myRow * S + u ];
+         const A a = sv[ wave ][ buf ][ myRow * S + u ];
+#pragma unroll
+         for( int i = 0; i < VW; i++ )
+            sum[ i ] = c >= 0 ? mulAddExact( sum[ i ], a, (A) g.x[ u ][ i ] ) : sum[ i ];
+      }
+      const int32_t len = sn[ wave ][ buf ][ myRow ];
+      if( len > S ) {
+         for( int32_t l = S; l < len; l++ ) {
+            const int64_t e = view.global( (int32_t) r, l );
+            const int32_t c = col[ e ];
+            if( c >= 0 ) {
+               const A a = toCompute( val[ e ], A() );
+               const VY xv = *reinterpret_cast< const VY* >( xs + (int64_t) c * k );
+#pragma unroll
+               for( int i = 0; i < VW; i++ )
+                  sum[ i ] = mulAddExact( sum[ i ], a, (A) xv[ i ] );
+            }
+         }
+      }
+      if( ! mine || r >= last )
+         return;
+      VY o;
+#pragma unroll
+      for( int i = 0; i < VW; i++ ) {
+         A v;
+         switch( mode ) {
+            case 0: v = sum[ i ]; break;
+            case 1: v = alpha * sum[ i ]; break;
+            case 2: v = beta * (A) g.y[ i ] + sum[ i ]; break;
+            default: v = beta * (A) g.y[ i ] + alpha * sum[ i ]; break;
+         }
+         o[ i ] = (Y) v;
+      }
+      Y* out = Yout + r * k + j0;
+      if( j0 == VW * jq )
+         *reinterpret_cast< VY* >( out ) = o;
+      else {
+#pragma unroll
+         for( int i = 0; i < VW; i++ )
+            if( j0 + i >= VW * jq )
+               out[ i ] = o[ i ];
+      }
+   };
+   // while a tile (base b0) is summed, X of the next (b1) is under way, the slots of the one after (b2)
+   // and the row starts of the one after that (b3) are loading
+   int64_t b0 = nextBase(), b1 = nextBase(), b2 = nextBase(), b3;
+   RowRun m = loadRun( b0 );
+   Slots s = loadSlots( m, b0 );
+   m = loadRun( b1 );
+   Gathered g0, g1;
+   share( 0, s );
+   s = loadSlots( m, b1 );
+   m = loadRun( b2 );
+   gather( 0, b0, g0 );
+   for( int t = 0; t < tiles; t += 2 ) {
+      b3 = nextBase();
+      share( 1, s );
+      s = loadSlots( m, b2 );
+      m = loadRun( b3 );
+      gather( 1, b1, g1 );
+      finish( 0, b0, g0 );
+      b0 = nextBase();
+      share( 0, s );
+      s = loadSlots( m, b3 );
+      m = loadRun( b0 );
+      gather( 0, b2, g0 );
+      finish( 1, b1, g1 );
+      b1 = b3;
+      const int64_t b4 = b0;
+      b0 = b2;
+      b2 = b4;
+   }
+}
+
+template< int L, int VW, typename V, typename A, typename Y, typename View >
+void launchMultiShort( const Matrix& M, const View& view, int32_t k, const Y* X, Y* Yv, double alpha, double beta,
+                       int32_t first, int32_t last, hipStream_t st )
+{
+   const int mode = beta == 0.0 ? ( alpha == 1.0 ? 0 : 1 ) : ( alpha == 1.0 ? 2 : 3 );
+   constexpr int RW = kWave / L;
+   constexpr int kWaves = 256 / kWave;
+   const int64_t all = ( (int64_t) last - first + RW - 1 ) / RW;
+   // X of one tile past a wave's last is gathered for nothing: many tiles a wave where there are enough
+   const int64_t tiles = all >= kMultiManyTiles ? 8 : 2;
+   const int64_t perBlock = tiles * kWaves;
+   int64_t blocks = ( all + perBlock - 1 ) / perBlock;
+   const int64_t chunk = multiChunk( M, blocks, perBlock * RW, (int64_t) k * sizeof( Y ) );
+   blocks = ( blocks + kXcds * chunk - 1 ) / ( kXcds * chunk ) * ( kXcds * chunk );
+   TNLHIP_REQUIRE( blocks < ( 1ll << 31 ), "too many rows for one launch" );
+   multiShortKernel< L, VW, V, A, Y ><<< (unsigned) blocks, 256, 0, st >>>(
+      view, M.columns.ptr, reinterpret_cast< const V* >( M.values.ptr ), k, X, Yv, (A) alpha, (A) beta, mode, first,
+      last, M.cols, (int32_t) chunk, (int32_t) tiles );
+   TNLHIP_CHECK( hipGetLastError() );
+}
+
+// Takes the product of short rows where it is the faster one; false: it is the other kernel's.  us, other kernel /
+// this one, SlicedEllpack: FP64 on the 128^3 Laplacian k = 3 97 / 62, 4 67 / 63, 7 196 / 114, 8 127 / 115,
+// 12 227 / 177, 16 239 / 209, 32 474 / 403; on the 1400^2 one k = 4 40 / 57, 8 114 / 101, 16 221 / 179; on
+// the 64^3 one k = 7 22.5 / 18.8, 8 14.3 / 18.7, 16 23.5 / 25.8.  FP32 128^3 k = 7 111 / 62, 8 41 / 58,
+// 16 110 / 110; CSRScalar FP64 k = 3 on 127 x 150 x 93 67 / 69, FP32 k = 3 on 128^3 43 / 61.  So it
+// takes the widths that 16-byte lanes do not divide (k = 3 only where FP64 slots lie slice by slice, from a
+// million rows on), and from four lanes a row (two FP64 columns each) on where there are rows enough to
+// walk.
+template< int KP, typename V, typename A, typename Y >
+bool launchShort( const Matrix& M, int32_t k, const Y* X, Y* Yv, double alpha, double beta, int32_t first, int32_t last,
+                  bool wide, hipStream_t st )
+{
+   constexpr int VW = KP <= 2 ? 2 : std::min( 16 / (int) sizeof( Y ), KP / 2 );
+   constexpr int L = KP / VW;
+   const int64_t rows = (int64_t) last - first;
+   if( wide && ( sizeof( Y ) != 8 || L < 4 || rows * L / kWave < kMultiManyTiles ) )
+      return false;
+   if( KP == 4 && ( sizeof( Y ) != 8 || kindOf( M.format ) == KIND_CSR || rows < 1000000 ) )
+      return false;
+   if constexpr( L >= 2 ) {
+      if( M.cols == 0 || M.meta.allocated > (int64_t) kMultiChunk * M.rows )
+         return false;
+      bool taken = false;
+      withView( M, [ & ]( auto view ) {
+         if constexpr( kRunView< decltype( view ) > ) {
+            launchMultiShort< L, VW, V, A, Y >( M, view, k, X, Yv, alpha, beta, first, last, st );
+            taken = true;
+         }
+      } );
+      return taken;
+   }
+   return false;
 }
 
 // 16-byte lanes (two FP64 or four FP32 columns) when k allows them and X, Y are 16-byte aligned
@@ -152,8 +454,11 @@ void launchMulti( const Matrix& M, int32_t k, const Y* X, Y* Yv, double alpha, d
 {
    constexpr int VW = 16 / (int) sizeof( Y ) < KP ? 16 / (int) sizeof( Y ) : KP;
    const bool aligned = ( ( reinterpret_cast< uintptr_t >( X ) | reinterpret_cast< uintptr_t >( Yv ) ) % 16 ) == 0;
+   const bool wide = VW > 1 && k % VW == 0 && aligned;
+   if( launchShort< KP, V, A, Y >( M, k, X, Yv, alpha, beta, first, last, wide, st ) )
+      return;
    if constexpr( VW > 1 ) {
-      if( k % VW == 0 && aligned ) {
+      if( wide ) {
          launchMultiW< KP, VW, V, A, Y >( M, k, X, Yv, alpha, beta, first, last, st );
          return;
       }
