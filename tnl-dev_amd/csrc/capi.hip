@@ -152,21 +152,29 @@ tnlhip_matrix_s* buildFromSegments( int format, int dtype, int32_t rows, int32_t
    // 70 -> 72 us and FP32 Ellpack 49.4 -> 52.1 us, so those keep the plain order
    if( ( format == TNLHIP_CHUNKED_ELLPACK || format == TNLHIP_SLICED_ELLPACK ) && dtype != TNLHIP_F64 )
       M->xcdRemap = 1;
-   // FP64 Ellpack: each XCD strides over its own eighth of the row blocks (distribution 3):
-   // 160^3, three alternated runs on one box, 78.4 -> 76.1 us; the other FP64 formats measured
-   // slower with an XCD split (SlicedEllpack 75.9 -> 79.1, CSRScalar 79.7 -> 82.9, CSRAdaptive
-   // 82.4 -> 84.9, ChunkedEllpack 72.0 -> 75.1 us) and keep the plain grid-stride
-   if( format == TNLHIP_ELLPACK && ( dtype == TNLHIP_F64 || dtype == TNLHIP_F32 ) )
-      M->xcdRemap = 3;  // FP32 with 32 workgroups per CU, below: 51.5 -> 50.3 us
-   // FP64 launch shapes from a sweep of workgroups per CU (8-64) and one or two rows per lane at
-   // 160^3 (two alternated runs): Ellpack 32 workgroups per CU, 76.6 -> 73.7 us; SlicedEllpack two
-   // rows per lane and 32 workgroups per CU, 76.1 -> 73.2 us (each row still summed left to right by
-   // one lane, so the bits do not change)
-   if( format == TNLHIP_ELLPACK && ( dtype == TNLHIP_F64 || dtype == TNLHIP_F32 ) )
+   // Row distribution and rows per lane of the padded formats, from a sweep of both and of 8 to 64
+   // workgroups per CU over Laplacians of 100^3, 127 x 150 x 93, 160^3 and 2000^2 rows (us; each row is summed
+   // left to right by one lane in all of them, so the bits do not change).  Two rows per lane and 32
+   // workgroups per CU suit all but FP32 SlicedEllpack:
+   //   SlicedEllpack FP64  one row, plain order 23.1 38.2 75.6 59.5; two rows 20.6 33.3 69.6 51.6, in XCD
+   //                       order 18.7 33.9 71.7 52.9 (taken up to 1.5 million rows)
+   //   SlicedEllpack FP32  one row, XCD order, 16 per CU 13.2 21.8 46.8 36.1
+   //   SlicedEllpack BF16  one row, XCD order 12.3 34.0 66.9 52.4; two rows, XCD order 12.2 20.5 44.9 32.8
+   //   Ellpack FP64        one row, each XCD striding over its eighth 23.5 41.5 73.5 60.7; two rows, XCD
+   //                       order 17.9 33.1 70.8 53.8
+   //   Ellpack FP32        the same 16.8 28.8 50.3 41.5 and 13.7 23.2 51.3 38.3 (taken up to 3 million rows)
+   //   Ellpack BF16        one row, plain order 14.0 35.5 83.0 60.2; two rows, XCD order 11.4 19.4 41.5 32.6
+   const bool sliced = format == TNLHIP_SLICED_ELLPACK;
+   if( ( sliced && dtype != TNLHIP_F32 ) || format == TNLHIP_ELLPACK ) {
       M->blocksPerCu = 32;
-   if( format == TNLHIP_SLICED_ELLPACK && dtype == TNLHIP_F64 ) {
       M->pairRows = 1;
-      M->blocksPerCu = 32;
+      M->xcdRemap = 1;
+      if( sliced && dtype == TNLHIP_F64 && rows > 1500000 )
+         M->xcdRemap = 0;
+      if( format == TNLHIP_ELLPACK && dtype == TNLHIP_F32 && rows > 3000000 ) {
+         M->pairRows = 0;
+         M->xcdRemap = 3;
+      }
    }
    if( format == TNLHIP_CSR_LIGHT )
       M->lanes = lightLanes( capTotal, rows );

@@ -64,7 +64,7 @@ __global__ void scatterFromCsrKernel( int32_t n, const int32_t* __restrict__ rp,
    }
    for( int o = kWave / 2; o > 0; o /= 2 )
       reach = max( reach, __shfl_xor( reach, o, kWave ) );
-   if( threadIdx.x % kWave == 0 && reach > 0 )
+   if( threadIdx.x % kWave == 0 && reach > __builtin_nontemporal_load( info + 1 ) )
       atomicMax( info + 1, reach );
 }
 

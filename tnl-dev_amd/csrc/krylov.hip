@@ -12,6 +12,7 @@ template< typename A, typename Y, typename Op >
 struct FusedKeeper
 {
    static constexpr bool kPlain = false;
+   static constexpr bool kStored = Op::kStored;
    Op op;
    const Y* diag;
    Y* y;

@@ -337,6 +337,7 @@ template< typename T >
 struct CgDirectionOperand
 {
    static constexpr int kSums = 1;
+   static constexpr bool kStored = false;
    const T* z;
    const T* pOld;
    T* p;
@@ -369,6 +370,7 @@ template< typename T >
 struct DotOperand : OpenGate
 {
    static constexpr int kSums = 1;
+   static constexpr bool kStored = true;
    const T* w;
    __device__ __forceinline__ T at( const T* x, int64_t c ) const { return x[ c ]; }
    __device__ __forceinline__ void row( int64_t r, T v, double ( &acc )[ 1 ] ) const
@@ -382,6 +384,7 @@ template< typename T >
 struct DotSquareOperand : OpenGate
 {
    static constexpr int kSums = 2;
+   static constexpr bool kStored = true;
    const T* s;
    __device__ __forceinline__ T at( const T* x, int64_t c ) const { return x[ c ]; }
    __device__ __forceinline__ void row( int64_t r, T v, double ( &acc )[ 2 ] ) const
@@ -396,6 +399,7 @@ template< typename T >
 struct BiDirectionOperand
 {
    static constexpr int kSums = 1;
+   static constexpr bool kStored = false;
    const T* r;
    const T* pOld;
    const T* ApOld;
@@ -422,6 +426,7 @@ template< typename T >
 struct BiSOperand
 {
    static constexpr int kSums = 2;
+   static constexpr bool kStored = false;
    const T* r;
    const T* Ap;
    T* s;

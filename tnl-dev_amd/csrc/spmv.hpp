@@ -16,6 +16,7 @@ template< typename A, typename Y >
 struct Keeper
 {
    static constexpr bool kPlain = true;
+   static constexpr bool kStored = true;  // the operand is a stored vector
    Y* y;
    A alpha, beta;
    const Y* diag;

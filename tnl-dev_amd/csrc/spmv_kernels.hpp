@@ -55,6 +55,18 @@ __device__ __forceinline__ bf16 ldnt( const bf16* p )
    return __ushort_as_bfloat16( __builtin_nontemporal_load( reinterpret_cast< const unsigned short* >( p ) ) );
 }
 
+// Whether a kernel leaves out the loads of a chunk that lie beyond the end of its rows (by branches that
+// whole waves or lane pairs take) instead of re-reading the last slot: from `least` value bytes on.  The
+// branches keep narrow loads from being issued together.  us, re-read / left out, at 160^3 and 2000^2:
+// staged CSR FP64 76.9 61.6 / 74.9 53.8, FP32 56.9 43.0 / 57.4 40.2, BF16 52.5 40.0 / 69.5 48.9;
+// CSRAdaptive FP64 79.9 57.7 / 78.0 56.5, FP32 61.9 43.7 / 60.9 42.1, BF16 56.9 39.4 / 71.2 51.3;
+// ChunkedEllpack FP64 71.1 59.6 / 68.5 54.0, FP32 46.3 38.4 / 50.3 38.4; BiEllpack FP64 77.1 68.7 / 72.1 56.3,
+// FP32 48.9 47.1 / 46.5 41.3, BF16 42.3 42.6 / 58.6 49.1.
+// An operand that is formed where it is gathered keeps the straight line (64^3 CG, SlicedEllpack: 14.8 us per iteration
+// against 18.0).
+template< typename V, typename Keep, int least >
+constexpr bool kSkipSlots = Keep::kStored && (int) sizeof( V ) >= least;
+
 __device__ __forceinline__ int64_t logicalBlock( int remap )
 {
    return logicalBlockOf( blockIdx.x, gridDim.x, remap );
@@ -200,9 +212,13 @@ __device__ __forceinline__ void csrScalarStagedRows( const int32_t* __restrict__
    auto loadRound = [ & ]( int32_t e0 ) {
 #pragma unroll
       for( int k = 0; k < kStageLoads; k++ ) {
-         const int32_t g = min( e0 + lane + k * kWave, size - 1 );
-         c[ k ] = ldnt( col + b + g );
-         v[ k ] = ldnt( val + b + g );
+         c[ k ] = -1;
+         v[ k ] = V( 0.0f );
+         if( ! kSkipSlots< V, Keep, 8 > || e0 + k * kWave < size ) {  // uniform over the wave
+            const int32_t g = min( e0 + lane + k * kWave, size - 1 );
+            c[ k ] = ldnt( col + b + g );
+            v[ k ] = ldnt( val + b + g );
+         }
       }
    };
    if constexpr( ! Keep::kPlain ) {
@@ -331,14 +347,21 @@ __global__ __launch_bounds__( 256 ) void csrAdaptiveKernel( int32_t nblocks, con
          V v[ kStageLoads ];
 #pragma unroll
          for( int k = 0; k < kStageLoads; k++ ) {
-            const int32_t e = min( e0 + lane + k * kWave, size - 1 );
-            c[ k ] = ldnt( col + b + e );
-            v[ k ] = ldnt( val + b + e );
+            c[ k ] = -1;
+            v[ k ] = V( 0.0f );
+            if( ! kSkipSlots< V, Keep, 4 > || e0 + k * kWave < size ) {  // uniform over the wave
+               const int32_t e = min( e0 + lane + k * kWave, size - 1 );
+               c[ k ] = ldnt( col + b + e );
+               v[ k ] = ldnt( val + b + e );
+            }
          }
          Y xv[ kStageLoads ];
 #pragma unroll
-         for( int k = 0; k < kStageLoads; k++ )
-            xv[ k ] = keep.at( x, c[ k ] < 0 ? 0 : c[ k ] );
+         for( int k = 0; k < kStageLoads; k++ ) {
+            xv[ k ] = Y( 0 );
+            if( ! kSkipSlots< V, Keep, 4 > || e0 + k * kWave < size )
+               xv[ k ] = keep.at( x, c[ k ] < 0 ? 0 : c[ k ] );
+         }
 #pragma unroll
          for( int k = 0; k < kStageLoads; k++ ) {
             const int32_t e = e0 + lane + k * kWave;
@@ -458,7 +481,10 @@ __device__ __forceinline__ int2 ldnt2( const int32_t* p )
    return make_int2( (int32_t) ( v & 0xffffffff ), (int32_t) ( v >> 32 ) );
 }
 
-// One or two (PAIR) rows per lane.  Slot index of row r at local index l: base( r ) + step * l.
+// One or two (PAIR) rows per lane.  A chunk's slots beyond the row's width are neither loaded nor
+// gathered (whole waves skip them): re-reading the last slot instead, as a lane pair did before, cost
+// a 5-wide row 3 of 8 loads (FP64 SlicedEllpack 160^3 77.1 -> 69.6 us, 128^3 41.2 -> 37.0, 2000^2 69.9 ->
+// 51.6).  Slot index of row r at local index l: base( r ) + step * l.
 template< bool PAIR, typename V, typename A, typename Y, typename Keep, typename Slots >
 __device__ __forceinline__ void paddedRows( const Slots& slots, const int32_t* __restrict__ col,
                                             const V* __restrict__ val, const Y* __restrict__ x, Keep& keep,
@@ -518,14 +544,19 @@ __device__ __forceinline__ void paddedRows( const Slots& slots, const int32_t* _
    }
    // a fused product's first chunk is loaded before begin()
    constexpr bool kAhead = PAIR && ! Keep::kPlain;
+   constexpr bool kSkip = kSkipSlots< V, Keep, 1 >;
    int2 c[ kChunk ];
    typename Pair< V >::T v[ kChunk ];
    auto loadChunk = [ & ]( int64_t b, int32_t l0, int32_t width, int64_t step ) {
 #pragma unroll
       for( int j = 0; j < kChunk; j++ ) {
-         const int64_t g = b + step * min( l0 + j, width - 1 );
-         c[ j ] = ldnt2( col + g );
-         v[ j ] = ldnt2( val + g );
+         c[ j ] = make_int2( -1, -1 );
+         v[ j ] = typename Pair< V >::T{};
+         if( ! kSkip || l0 + j < width ) {
+            const int64_t g = b + step * ( kSkip ? l0 + j : min( l0 + j, width - 1 ) );
+            c[ j ] = ldnt2( col + g );
+            v[ j ] = ldnt2( val + g );
+         }
       }
    };
    bool ahead = false;
@@ -550,16 +581,19 @@ __device__ __forceinline__ void paddedRows( const Slots& slots, const int32_t* _
             Y x0[ kChunk ], x1[ kChunk ];
 #pragma unroll
             for( int j = 0; j < kChunk; j++ ) {
-               x0[ j ] = keep.at( x, c[ j ].x < 0 ? 0 : c[ j ].x );
-               x1[ j ] = keep.at( x, c[ j ].y < 0 ? 0 : c[ j ].y );
+               x0[ j ] = x1[ j ] = Y( 0 );
+               if( ! kSkip || l0 + j < width ) {
+                  x0[ j ] = keep.at( x, c[ j ].x < 0 ? 0 : c[ j ].x );
+                  x1[ j ] = keep.at( x, c[ j ].y < 0 ? 0 : c[ j ].y );
+               }
             }
 #pragma unroll
             for( int j = 0; j < kChunk; j++ ) {
                V a, bb;
                split( v[ j ], a, bb );
-               if( l0 + j < width && c[ j ].x >= 0 )
+               if( ( kSkip || l0 + j < width ) && c[ j ].x >= 0 )
                   s0 = mulAddExact( s0, toCompute( a, A() ), (A) x0[ j ] );
-               if( l0 + j < width && c[ j ].y >= 0 )
+               if( ( kSkip || l0 + j < width ) && c[ j ].y >= 0 )
                   s1 = mulAddExact( s1, toCompute( bb, A() ), (A) x1[ j ] );
             }
          }
@@ -674,17 +708,25 @@ __global__ __launch_bounds__( 256 ) void chunkedKernel( int32_t nslices, const i
          V v[ kChunk ];
 #pragma unroll
          for( int j = 0; j < kChunk; j++ ) {
-            const int64_t g = (int64_t) s.w + t + (int64_t) kChunksInSlice * min( k0 + j, s.y - 1 );
-            c[ j ] = ldnt( col + g );
-            v[ j ] = ldnt( val + g );
+            c[ j ] = -1;
+            v[ j ] = V( 0.0f );
+            if( ! kSkipSlots< V, Keep, 8 > || k0 + j < s.y ) {  // uniform over the workgroup
+               const int32_t l = kSkipSlots< V, Keep, 8 > ? k0 + j : min( k0 + j, s.y - 1 );
+               const int64_t g = (int64_t) s.w + t + (int64_t) kChunksInSlice * l;
+               c[ j ] = ldnt( col + g );
+               v[ j ] = ldnt( val + g );
+            }
          }
          Y xv[ kChunk ];
 #pragma unroll
-         for( int j = 0; j < kChunk; j++ )
-            xv[ j ] = keep.at( x, c[ j ] < 0 ? 0 : c[ j ] );
+         for( int j = 0; j < kChunk; j++ ) {
+            xv[ j ] = Y( 0 );
+            if( ! kSkipSlots< V, Keep, 8 > || k0 + j < s.y )
+               xv[ j ] = keep.at( x, c[ j ] < 0 ? 0 : c[ j ] );
+         }
 #pragma unroll
          for( int j = 0; j < kChunk; j++ )
-            if( k0 + j < s.y && c[ j ] >= 0 )
+            if( ( kSkipSlots< V, Keep, 8 > || k0 + j < s.y ) && c[ j ] >= 0 )
                p += toCompute( v[ j ], A() ) * (A) xv[ j ];
          // the last slot read is padding: so is the rest of this lane's chunk
          if( stopAtPadding && __all( c[ kChunk - 1 ] < 0 ) )
@@ -766,17 +808,24 @@ __global__ __launch_bounds__( 256 ) void biellpackKernel( int32_t n, int32_t str
                V v[ kBiUnroll ];
 #pragma unroll
                for( int j = 0; j < kBiUnroll; j++ ) {
-                  const int32_t e = min( e0 + j * kStrip, size - 1 );
-                  c[ j ] = ldnt( col + base + e );
-                  v[ j ] = ldnt( val + base + e );
+                  c[ j ] = -1;
+                  v[ j ] = V( 0.0f );
+                  if( ! kSkipSlots< V, Keep, 4 > || e0 + j * kStrip < size ) {
+                     const int32_t e = kSkipSlots< V, Keep, 4 > ? e0 + j * kStrip : min( e0 + j * kStrip, size - 1 );
+                     c[ j ] = ldnt( col + base + e );
+                     v[ j ] = ldnt( val + base + e );
+                  }
                }
                Y xv[ kBiUnroll ];
 #pragma unroll
-               for( int j = 0; j < kBiUnroll; j++ )
-                  xv[ j ] = keep.at( x, c[ j ] < 0 ? 0 : c[ j ] );
+               for( int j = 0; j < kBiUnroll; j++ ) {
+                  xv[ j ] = Y( 0 );
+                  if( ! kSkipSlots< V, Keep, 4 > || e0 + j * kStrip < size )
+                     xv[ j ] = keep.at( x, c[ j ] < 0 ? 0 : c[ j ] );
+               }
 #pragma unroll
                for( int j = 0; j < kBiUnroll; j++ )
-                  if( e0 + j * kStrip < size && c[ j ] >= 0 )
+                  if( ( kSkipSlots< V, Keep, 4 > || e0 + j * kStrip < size ) && c[ j ] >= 0 )
                      p += toCompute( v[ j ], A() ) * (A) xv[ j ];
             }
             for( int o = h; o < kStrip; o <<= 1 )
@@ -928,7 +977,10 @@ unsigned launchProduct( const Matrix& M, const Y* x, Keep keep, int32_t first, i
          // with slice size 1 has no such neighbours (row r + 1 lies in the next slice), so it
          // takes one row per lane whatever pair_rows says
          const bool pair = M.pairRows != 0 && ( M.format == TNLHIP_ELLPACK || M.meta.sliceSize >= 2 );
-         if( ! knownDistribution( M.xcdRemap ) )
+         // a fused product takes the rows in the order of the passes around it, which read and write the same
+         // vectors: 64^3 CG 14.8 us per iteration against 17.1 in XCD order
+         const int dist = Keep::kPlain ? M.xcdRemap : 0;
+         if( ! knownDistribution( dist ) )
             throw Error( TNLHIP_ERROR_INVALID_ARGUMENT, "unknown row distribution" );
          const PaddedLaunch pl = paddedLaunch( first, last, pair, M.blocksPerCu, deviceProps().cus );
          const unsigned grid = (unsigned) pl.grid;
@@ -938,18 +990,18 @@ unsigned launchProduct( const Matrix& M, const Y* x, Keep keep, int32_t first, i
          if( M.format == TNLHIP_ELLPACK ) {
             if( pair )
                run( ellpackKernel< true, V, A, Y, Keep >, grid, es, col, val, x, keep, first, last, (int32_t) per,
-                    M.xcdRemap );
+                    dist );
             else
                run( ellpackKernel< false, V, A, Y, Keep >, grid, es, col, val, x, keep, first, last, (int32_t) per,
-                    M.xcdRemap );
+                    dist );
          }
          else {
             if( pair )
                run( slicedKernel< true, V, A, Y, Keep >, grid, ss, col, val, x, keep, first, last, (int32_t) per,
-                    M.xcdRemap );
+                    dist );
             else
                run( slicedKernel< false, V, A, Y, Keep >, grid, ss, col, val, x, keep, first, last, (int32_t) per,
-                    M.xcdRemap );
+                    dist );
          }
          break;
       }
