@@ -358,20 +358,28 @@ void resetState( SolverImpl& S )
 // same polynomial on every call), so it preconditions GMRES, BiCGStab and TFQMR as Jacobi does
 // and, for symmetric P, CG.  Each step is one product whose keeper does the update; the steps
 // alternate between `out` and a work vector so that the last one lands in `out`.
+// z_j's buffer: the last one, z_k, is `out`
 template< typename T >
-void polyApplyTyped( SolverImpl& S, const void* in, void* out, Gate gate )
+T* polyBuffer( SolverImpl& S, void* out, int j )
+{
+   return ( S.params.poly_degree - j ) % 2 == 0 ? (T*) out : (T*) S.polyVecs.ptr + S.ld;
+}
+
+// `started`: z_0 is in its buffer already
+template< typename T >
+void polyApplyTyped( SolverImpl& S, const void* in, void* out, Gate gate, bool started = false )
 {
    const Matrix& P = S.polyMatrix ? *S.polyMatrix : *S.A;
    T* sv = (T*) S.polyVecs.ptr;
-   T* tv = sv + S.ld;
    const T* src = (const T*) in;
    if( in == out ) {
       launchElementwise( S.n, OpCopy< T >{ {}, sv, src }, gate, S.stream );
       src = sv;
    }
    const int k = S.params.poly_degree;
-   auto buf = [ & ]( int j ) { return ( ( k - j ) % 2 == 0 ) ? (T*) out : tv; };
-   launchElementwise( S.n, OpDivide< T >{ {}, buf( 0 ), src, (const T*) S.diag.ptr }, gate, S.stream );
+   auto buf = [ & ]( int j ) { return polyBuffer< T >( S, out, j ); };
+   if( ! started )
+      launchElementwise( S.n, OpDivide< T >{ {}, buf( 0 ), src, (const T*) S.diag.ptr }, gate, S.stream );
    for( int j = 1; j <= k; j++ )
       spmvJacobiStepGated( P, buf( j - 1 ), buf( j ), src, S.diag.ptr, gate.flags, gate.mode, S.stream );
 }
@@ -392,9 +400,22 @@ void precSolve( SolverImpl& S, const void* in, void* out, Gate gate )
 void matvec( SolverImpl& S, const void* x, void* y, Gate gate )
 {
    if( S.params.preconditioner == 3 ) {
-      // A x into the polynomial's input vector, then the polynomial into y (no copy)
-      spmvLaunchGated( *S.A, x, S.polyVecs.ptr, 1.0, 0.0, nullptr, gate.flags, gate.mode, S.stream );
-      precSolve( S, S.polyVecs.ptr, y, gate );
+      // A x into the polynomial's input vector, then the polynomial into y (no copy); a general matrix's
+      // product writes z_0 = D^-1 A x beside it
+      const bool general = ! S.A->symmetric;
+      auto apply = [ & ]( auto* tag ) {
+         using T = std::remove_pointer_t< decltype( tag ) >;
+         if( general )
+            spmvQuotientGated( *S.A, x, S.polyVecs.ptr, polyBuffer< T >( S, y, 0 ), S.diag.ptr, gate.flags, gate.mode,
+                               S.stream );
+         else
+            spmvLaunchGated( *S.A, x, S.polyVecs.ptr, 1.0, 0.0, nullptr, gate.flags, gate.mode, S.stream );
+         polyApplyTyped< T >( S, S.polyVecs.ptr, y, gate, general );
+      };
+      if( S.vdtype == TNLHIP_F64 )
+         apply( (double*) nullptr );
+      else
+         apply( (float*) nullptr );
       return;
    }
    spmvLaunchGated( *S.A, x, y, 1.0, 0.0, S.params.preconditioner == 1 ? S.diag.ptr : nullptr, gate.flags, gate.mode,
@@ -1938,19 +1959,19 @@ struct FinGmresCycleStart
    State* st;
    Small q;
    bool cwy;
-   __device__ void operator()() const
+   __device__ void operator()( int lane ) const
    {
-      for( int k = 0; k < ( q.m + 1 ) * q.m; k++ )
+      for( int k = lane; k < ( q.m + 1 ) * q.m; k += kWave )
          q.H[ k ] = 0.0;
-      for( int k = 0; k <= q.m; k++ )
-         q.s[ k ] = 0.0;
+      for( int k = lane; k <= q.m; k += kWave )
+         q.s[ k ] = k == 0 && ! cwy ? st->beta_gm : 0.0;
       if( cwy )
-         for( int k = 0; k < ( q.mx + 1 ) * ( q.mx + 1 ); k++ )
+         for( int k = lane; k < ( q.mx + 1 ) * ( q.mx + 1 ); k += kWave )
             q.T[ k ] = 0.0;
-      else
-         q.s[ 0 ] = st->beta_gm;
-      st->o_steps = q.m;
-      st->flags[ 0 ] = 0;
+      if( lane == 0 ) {
+         st->o_steps = q.m;
+         st->flags[ 0 ] = 0;
+      }
    }
 };
 
@@ -2302,26 +2323,6 @@ struct FinYL
    }
 };
 
-struct FinTUpdate
-{
-   // [T_i]_{0..i-1} = - T_{i-1} * t_i * aux
-   Small q;
-   int i;
-   static constexpr bool kLaneParallel = true;
-   __device__ void operator()( const double* aux, int k ) const
-   {
-      // entry k of the new column, one lane each (reads columns < i only)
-      const int mx = q.mx;
-      const double ti = q.T[ i + i * ( mx + 1 ) ];
-      if( k < i ) {
-         double t = 0.0;
-         for( int j = k; j < i; j++ )
-            t -= q.T[ k + j * ( mx + 1 ) ] * ( ti * aux[ j ] );
-         q.T[ k + i * ( mx + 1 ) ] = t;
-      }
-   }
-};
-
 struct FinCwyAux
 {
    // aux = T_i * Y_i^T e_i  (from YL)
@@ -2487,44 +2488,112 @@ struct OpCwyZGenerate
    }
 };
 
-// The rest of hauseholder_generate for step i from the fused sums: y_ii +- |y|, t_i, and the
-// new column of T from Y^T y_i corrected for the changed entry i (GMRES.hpp:464-520).
+// The scalar work of CWY step i >= 1, by one workgroup, in front of the step's passes:
+//   - hauseholder_generate's finish from the fused sums: y_ii +- |y|, t_i, and the new column of T from
+//     Y^T y_i corrected for the changed entry i (GMRES.hpp:464-520);
+//   - hauseholder_apply_trunc: YL_i and column i - 1 of H;
+//   - aux = T_i Y_i^T e_i, the coefficients of v = e_i - Y_i aux;
+//   - the end of step i (Givens rotation of column i - 1, residue, stopping rule) and, for i < m, the top of
+//     step i + 1 (FinGmresStepEnd, FinGmresStepStart).  They depend on nothing that the step's passes make, so a
+//     stop here leaves those out.
+// Everything the parts read is loaded into LDS at once, beside the partial sums: as a chain of device-memory
+// loads they took 13.8 us and another launch's 6.6 us (32 columns, FP64).  The Givens chain runs on the second
+// wavefront beside the column of T.
 template< typename T, int C >
-struct FinGenerateFused
+__global__ __launch_bounds__( kReduceBlock ) void cwyStepKernel( State* state, Small q, T* yi, const T* z, int i, int64_t n,
+                                                                 Stop stop, double* hist, int64_t cap, ReduceSlot slot,
+                                                                 int grid, Gate gate )
 {
-   Small q;
-   T* yi;
-   const T* Y;
-   int64_t ld;
-   int i;
-   static constexpr bool kLaneParallel = true;
-   __device__ void operator()( const double* v, int lane ) const
-   {
-      __shared__ double aux[ kMaxMulti ];
-      __shared__ double delta;
-      const int mx = q.mx;
-      if( lane == 0 ) {
-         const double normz = sqrt( v[ C - 1 ] );
-         const double y_ii = (double) yi[ i ];
-         const T ynew = (T) ( y_ii > 0.0 ? y_ii + normz : y_ii - normz );
-         yi[ i ] = ynew;
-         const double norm_yi_squared = 2 * ( normz * normz + fabs( y_ii ) * normz );
-         q.T[ i + i * ( mx + 1 ) ] = 2.0 / norm_yi_squared;
-         delta = (double) ynew - y_ii;
-      }
-      __syncthreads();
-      if( lane < i )
-         aux[ lane ] = v[ lane ] + (double) Y[ i + (int64_t) lane * ld ] * delta;
-      __syncthreads();
-      const double ti = q.T[ i + i * ( mx + 1 ) ];
-      if( lane < i ) {
-         double t = 0.0;
-         for( int j = lane; j < i; j++ )
-            t -= q.T[ lane + j * ( mx + 1 ) ] * ( ti * aux[ j ] );
-         q.T[ lane + i * ( mx + 1 ) ] = t;
-      }
+   __shared__ double Ts[ kMaxMulti * kMaxMulti ];  // column j < i of T at j * kMaxMulti
+   __shared__ double yk[ kMaxMulti ];              // y_k[ i ], k <= i
+   __shared__ double ys[ kMaxMulti ], zs[ kMaxMulti ], cs[ kMaxMulti ], sn[ kMaxMulti ], Hc[ kMaxMulti + 1 ];
+   __shared__ double aux[ kMaxMulti ], tot[ C ];
+   __shared__ double ti, ynew, delta;
+   const int t = threadIdx.x;
+   const int m = q.m, mx = q.mx, m1 = mx + 1;
+   const bool open = gate.open();
+   for( int e = t; e < i * kMaxMulti; e += kReduceBlock ) {
+      const int j = e / kMaxMulti, k = e % kMaxMulti;
+      Ts[ e ] = k <= j ? q.T[ k + j * m1 ] : 0.0;
    }
-};
+   if( t < i ) {
+      yk[ t ] = q.YL[ i + t * m1 ];
+      cs[ t ] = q.cs[ t ];
+      sn[ t ] = q.sn[ t ];
+   }
+   if( t <= mx )
+      ys[ t ] = t < n ? (double) yi[ t ] : 0.0;
+   if( t <= i )
+      zs[ t ] = t < n ? (double) z[ t ] : 0.0;
+   const double sPrev = q.s[ i - 1 ], sThis = q.s[ i ];
+   const double normb = state->normb;
+   const int32_t it = state->it, histLen = state->histLen;
+   if( ! open )  // uniform over the workgroup
+      return;
+   sumPartials< C >( slot, grid, tot );  // ends with a barrier
+   if( t == 0 ) {
+      const double normz = sqrt( tot[ C - 1 ] );
+      const double y_ii = ys[ i ];
+      const T yn = (T) ( y_ii > 0.0 ? y_ii + normz : y_ii - normz );
+      yi[ i ] = yn;
+      ynew = (double) yn;
+      ti = 2.0 / ( 2 * ( normz * normz + fabs( y_ii ) * normz ) );
+      q.T[ i + i * m1 ] = ti;
+      delta = (double) yn - y_ii;
+   }
+   __syncthreads();
+   if( t <= mx )
+      q.YL[ t + i * m1 ] = t == i ? ynew : ys[ t ];
+   if( t < i )
+      aux[ t ] = tot[ t ] + yk[ t ] * delta;
+   if( t <= i )
+      Hc[ t ] = zs[ t ] - ( t == i ? ynew : ys[ t ] );
+   __syncthreads();
+   if( t == kWave ) {
+      // FinGmresStepEnd with Givens index i - 1, the rotations of column i - 1 in LDS
+      for( int k = 0; k < i - 1; k++ )
+         applyPlaneRotation( Hc[ k ], Hc[ k + 1 ], cs[ k ], sn[ k ] );
+      double sa = sPrev, sb = sThis;
+      if( Hc[ i ] != 0.0 ) {
+         double c1, s1;
+         generatePlaneRotation( Hc[ i - 1 ], Hc[ i ], c1, s1 );
+         applyPlaneRotation( Hc[ i - 1 ], Hc[ i ], c1, s1 );
+         applyPlaneRotation( sa, sb, c1, s1 );
+         q.cs[ i - 1 ] = c1;
+         q.sn[ i - 1 ] = s1;
+      }
+      for( int k = 0; k <= i; k++ )
+         q.H[ k + ( i - 1 ) * ( m + 1 ) ] = Hc[ k ];
+      q.s[ i - 1 ] = sa;
+      q.s[ i ] = sb;
+      State& s = *state;
+      const double r = fabs( sb ) / normb;
+      s.residue = r;
+      if( histLen < cap ) {
+         hist[ 2 * (int64_t) histLen ] = r;
+         hist[ 2 * (int64_t) histLen + 1 ] = (double) it;
+      }
+      s.histLen = histLen + 1;
+      if( isnan( r ) || it > stop.maxIt || ( r > stop.div && it >= stop.minIt ) || ( r < stop.conv && it >= stop.minIt ) ) {
+         s.o_steps = i - 1;
+         s.flags[ 0 ] = 1;
+      }
+      else if( i < m )
+         s.it = it + 1;  // the top of step i + 1: its check is the one just made
+   }
+   if( t < i ) {
+      double c = 0.0;
+      for( int j = t; j < i; j++ )
+         c -= Ts[ t + j * kMaxMulti ] * ( ti * aux[ j ] );
+      q.T[ t + i * m1 ] = c;
+      double a2 = 0.0;
+      for( int j = t; j < i; j++ )
+         a2 += Ts[ t + j * kMaxMulti ] * yk[ j ];
+      q.aux[ t ] = a2 + c * ynew;
+   }
+   else if( t == i )
+      q.aux[ t ] = ti * ynew;
+}
 
 template< typename T, int C >
 void launchCwyZGenerate( int64_t n, T* z, const T* w, const T* Y, int64_t ld, const double* aux, int count, Small q,
@@ -2535,35 +2604,13 @@ void launchCwyZGenerate( int64_t n, T* z, const T* w, const T* Y, int64_t ld, co
    TNLHIP_CHECK( hipGetLastError() );
 }
 
-// The generate finish, then apply_trunc and aux = T_i Y_i^T e_i, in one workgroup: every lane
-// calls each part (they hold workgroup barriers), parts are separated by barriers so each sees
-// the previous one's writes.
 template< typename T, int C >
-struct FinGenerateApplyAux
-{
-   FinGenerateFused< T, C > generate;
-   FinYL< T > applyTrunc;
-   FinCwyAux aux;
-   static constexpr bool kLaneParallel = true;
-   __device__ void operator()( const double* v, int lane ) const
-   {
-      generate( v, lane );
-      __syncthreads();
-      applyTrunc( lane );
-      __syncthreads();
-      aux( lane );
-   }
-};
-
-template< typename T, int C >
-void launchGenerateFinal( int64_t n, State* state, Small q, T* yi, const T* z, const T* Y, int64_t ld, int i,
-                          ReduceSlot slot, Gate gate, hipStream_t st )
+void launchCwyStep( State* state, Small q, T* yi, const T* z, int i, int64_t n, Stop stop, double* hist, int64_t cap,
+                    ReduceSlot slot, Gate gate, hipStream_t st )
 {
    // the partials of launchCwyZGenerate over the same n
-   reduceFinalKernel< C ><<< 1, kReduceBlock, 0, st >>>(
-      FinGenerateApplyAux< T, C >{ FinGenerateFused< T, C >{ q, yi, Y, ld, i }, FinYL< T >{ state, q, yi, z, i, n },
-                                   FinCwyAux{ q, i } },
-      slot, reduceGridFor( C, n ), gate );
+   cwyStepKernel< T, C ><<< 1, kReduceBlock, 0, st >>>( state, q, yi, z, i, n, stop, hist, cap, slot,
+                                                        reduceGridFor( C, n ), gate );
    TNLHIP_CHECK( hipGetLastError() );
 }
 
@@ -2653,7 +2700,7 @@ void solveGMRES( SolverImpl& S, const void* b, void* xv )
          }
       }
       q.m = m;
-      launchScalar( FinGmresCycleStart{ st, q, cwy }, always, S.stream );
+      launchWave( FinGmresCycleStart{ st, q, cwy }, always, S.stream );
       if( ! cwy ) {
          // v_0 = r / beta
          launchElementwise( n, OpScale< T >{ V, r, &st->beta_gm, true, 0 }, always, S.stream );
@@ -2705,15 +2752,15 @@ void solveGMRES( SolverImpl& S, const void* b, void* xv )
                launchReduce< 1 >( n, OpTruncate< T >{ {}, yi, z, i }, FinHouseholder< T >{ st, q, yi, i },
                                   S.ws.slot( 0 ), cycle, S.stream );
             else {
-               // with apply_trunc (s or H column i-1) and hauseholder_cwy's aux = T_i Y_i^T e_i
-               // (for v = e_i - Y_i aux) in the same launch
                const int C = fusedBucket( i );
                if( C == 8 )
-                  launchGenerateFinal< T, 8 >( n, st, q, yi, z, V, ld, i, S.ws.slot( 3 ), cycle, S.stream );
+                  launchCwyStep< T, 8 >( st, q, yi, z, i, n, stop, S.hist.ptr, S.histCap, S.ws.slot( 3 ), cycle, S.stream );
                else if( C == 16 )
-                  launchGenerateFinal< T, 16 >( n, st, q, yi, z, V, ld, i, S.ws.slot( 3 ), cycle, S.stream );
+                  launchCwyStep< T, 16 >( st, q, yi, z, i, n, stop, S.hist.ptr, S.histCap, S.ws.slot( 3 ), cycle, S.stream );
                else
-                  launchGenerateFinal< T, 32 >( n, st, q, yi, z, V, ld, i, S.ws.slot( 3 ), cycle, S.stream );
+                  launchCwyStep< T, 32 >( st, q, yi, z, i, n, stop, S.hist.ptr, S.histCap, S.ws.slot( 3 ), cycle, S.stream );
+               if( i == m )
+                  break;
             }
             // hauseholder_apply_trunc (s or H column i-1)
             // apply_trunc, then hauseholder_cwy's aux = T_i Y_i^T e_i (for v = e_i - Y_i aux)
@@ -2733,11 +2780,11 @@ void solveGMRES( SolverImpl& S, const void* b, void* xv )
                else
                   launchCwyZGenerate< T, 32 >( n, z, w, V, ld, q.aux, i + 1, q, S.ws.slot( 3 ), cycle, S.stream );
             }
-            const FinGmresStepEnd end{ st, q, stop, S.hist.ptr, S.histCap, i, i, i - 1, i > 0, i - 1, i > 0 };
-            if( i < m )
+            if( i == 0 ) {
+               // (later steps' ends and tops are cwyStepKernel's)
+               const FinGmresStepEnd end{ st, q, stop, S.hist.ptr, S.histCap, 0, 0, -1, false, -1, false };
                launchScalar( FinGmresStepEndThenStart{ end, FinGmresStepStart{ st, q, stop, -1 } }, cycle, S.stream );
-            else
-               launchScalar( end, cycle, S.stream );
+            }
          }
       }
       h = readState( S );

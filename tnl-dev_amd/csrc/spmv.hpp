@@ -11,7 +11,8 @@ namespace tnlhip {
 // SparseMatrixView.hpp:447-490: direct / alpha / beta / general keepers; mode 4 divides by
 // a diagonal, which fuses Preconditioners::Diagonal::solve (x = b / diag) into the product;
 // mode 5 is one step of the Jacobi splitting, y = prev + (rhs - v) / diag (the Jacobi-polynomial
-// preconditioner; y must not alias prev, which other rows gather).
+// preconditioner; y must not alias prev, which other rows gather); mode 6 stores v and v / diag (a
+// product and the start of the polynomial over it).
 template< typename A, typename Y >
 struct Keeper
 {
@@ -28,6 +29,7 @@ struct Keeper
    bool streamY = true;
    const Y* rhs = nullptr;   // mode 5
    const Y* prev = nullptr;  // mode 5
+   Y* y2 = nullptr;          // mode 6
    // the row kernels' other calls (spmv_kernels.hpp): a plain product has nothing to do there
    __device__ __forceinline__ void prefetch() {}
    __device__ __forceinline__ bool begin() { return true; }
@@ -50,6 +52,10 @@ struct Keeper
          case 2: out = beta * (A) y[ row ] + v; break;
          case 3: out = beta * (A) y[ row ] + alpha * v; break;
          case 4: out = v / (A) diag[ row ]; break;
+         case 6:
+            out = v;
+            y2[ row ] = (Y) ( v / (A) diag[ row ] );
+            break;
          default: out = (A) prev[ row ] + ( (A) rhs[ row ] - v ) / (A) diag[ row ]; break;
       }
       if( streamY )
