@@ -248,6 +248,44 @@ def test_bicgstab_restart_follows_the_oracle(tnl, dev, m, use_graph):
     assert abs(its - ref["iterations"]) <= 1 and ok == bool(ref["converged"])
 
 
+@pytest.mark.parametrize("restart", [1, 2, 6, 7, 8, 14, 15, 16, 30, 31])
+@pytest.mark.parametrize("n", [40, 257, 4913])
+def test_cwy_steps_follow_the_oracle(tnl, dev, restart, n):
+    # restart lengths around the column buckets of the step's sums (8, 16, 32); sizes about a workgroup
+    i = np.arange(n)
+    r = np.concatenate([i[1:], i, i[:-1]])
+    c = np.concatenate([i[1:] - 1, i, i[:-1] + 1])
+    v = np.concatenate([np.full(n - 1, -1.3), 2.5 + 0.2 * np.cos(i), np.full(n - 1, -0.8)])
+    o = np.lexsort((c, r))
+    rp = np.zeros(n + 1, np.int32)
+    np.cumsum(np.bincount(r, minlength=n), out=rp[1:])
+    b = W.uniform_vector(n, 3)
+    for pre in (0, 1):
+        p = dict(convergence_residue=1e-9, max_iterations=3 * restart + 2, preconditioner=pre, gmres_variant="CWY",
+                 restarting_min=restart, restarting_max=restart)
+        ref = O.solve("gmres", rp, c[o].astype(np.int32), v[o], b, **{**p, "gmres_variant": 4})
+        ok, its, _, h, x = _run_device_solver(tnl, dev, "gmres", rp, c[o].astype(np.int32), v[o], b, fmt="SlicedEllpack",
+                                              **p)
+        m = min(len(h), len(ref["history"]), 2 * restart + 2)
+        assert abs(len(h) - len(ref["history"])) <= 1 and abs(its - ref["iterations"]) <= 1
+        # Householder vectors keep the basis orthogonal to rounding: the sums' order shows at 1e-13 a step
+        np.testing.assert_allclose(h[:m], ref["history"][:m], rtol=1e-8, atol=1e-13)
+
+
+@pytest.mark.parametrize("fmt", ["CSRScalar", "CSRAdaptive", "Ellpack", "SlicedEllpack", "ChunkedEllpack", "BiEllpack"])
+@pytest.mark.parametrize("dt,degree", [("f64", 0), ("f64", 1), ("f64", 2), ("f32", 3)])
+def test_polynomial_start_in_the_product_of_every_format(tnl, dev, fmt, dt, degree):
+    # z_0 = D^-1 A v stored beside the product: every format's run follows the CSRScalar one
+    rp, c, v = W.convection_diffusion_3d(9, 10.0)
+    b = W.uniform_vector(len(rp) - 1, 4)
+    p = dict(dtype=dt, convergence_residue=1e-9 if dt == "f64" else 1e-4, max_iterations=200, preconditioner=3,
+             poly_degree=degree, restarting_min=10, restarting_max=10)
+    want = _run_device_solver(tnl, dev, "gmres", rp, c, v, b, fmt="CSRScalar", **p)
+    got = _run_device_solver(tnl, dev, "gmres", rp, c, v, b, fmt=fmt, **p)
+    assert got[0] and want[0] and abs(got[1] - want[1]) <= 1
+    np.testing.assert_allclose(got[3][:8], want[3][:8], rtol=1e-9 if dt == "f64" else 1e-3)
+
+
 @pytest.mark.parametrize("method", ["cg", "bicgstab"])
 @pytest.mark.parametrize("most", [0, 1, 2, 11, 12, 13, 29])
 def test_iteration_limits_of_fused_solves(tnl, dev, method, most):
