@@ -239,15 +239,21 @@ def _check(status):
         raise TnlHipError(status, msg)
 
 
+# Addresses and stream handles go to the library as plain integers (its argument types make pointers of
+# them): a small product's kernel is shorter than the objects around its call took to make (256^2: 7.4 us a
+# call with a c_void_p each, a Stream object and the type lookup per call).
 def _ptr(t):
-    return C.c_void_p(t.data_ptr()) if t is not None else C.c_void_p(0)
+    return t.data_ptr() if t is not None else 0
 
 
 def _stream(stream):
     if stream is None:
         import torch
-        return C.c_void_p(torch.cuda.current_stream().cuda_stream)
-    return C.c_void_p(stream if isinstance(stream, int) else stream.cuda_stream)
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        if raw is None or not torch.cuda.is_initialized():
+            return torch.cuda.current_stream().cuda_stream
+        return raw(torch.cuda.current_device())
+    return stream if isinstance(stream, int) else stream.cuda_stream
 
 
 def device_info():
@@ -277,6 +283,18 @@ class SparseMatrix:
         info = MatrixInfo()
         _check(lib.tnlhip_matrix_get_info(self._h, C.byref(info)))
         self.info = info
+
+    @property
+    def info(self):
+        return self._info
+
+    @info.setter
+    def info(self, info):
+        import torch
+        self._info = info
+        # what every product checks, read from the struct once
+        self._rows, self._columns = info.rows, info.columns
+        self._vector_dtype = {0: torch.float64, 3: torch.int32}.get(info.value_dtype, torch.float32)
 
     @classmethod
     def from_csr(cls, row_pointers, column_indexes, values, columns=None, format="CSRScalar", dtype="f64"):
@@ -395,8 +413,7 @@ class SparseMatrix:
 
     @property
     def vector_dtype(self):
-        import torch
-        return {0: torch.float64, 3: torch.int32}.get(self.info.value_dtype, torch.float32)
+        return self._vector_dtype
 
     def convert(self, format, dtype=None):
         """B = A into another format / value type, on the device."""
@@ -488,10 +505,10 @@ class SparseMatrix:
                       firstRow=0, lastRow=0, stream=None):
         """outVector = matrixMultiplicator * A inVector + outVectorMultiplicator * outVector over rows
         [firstRow, lastRow) (lastRow 0 = all), SparseMatrix.h:1078-1085.  Asynchronous on the stream."""
-        dt = self.vector_dtype
+        dt = self._vector_dtype
         if inVector.dtype != dt or outVector.dtype != dt:
             raise TypeError(f"vectors must be {dt}")
-        if inVector.numel() != self.info.columns or outVector.numel() != self.info.rows:
+        if inVector.numel() != self._columns or outVector.numel() != self._rows:
             raise ValueError("vector sizes do not match the matrix")
         _check(lib.tnlhip_spmv(self._h, _ptr(inVector), _ptr(outVector), float(matrixMultiplicator),
                                float(outVectorMultiplicator), int(firstRow), int(lastRow), _stream(stream)))
@@ -508,7 +525,7 @@ class SparseMatrix:
             raise ValueError("blocks of vectors are (size, k) tensors with the same k")
         if not (inVectors.is_contiguous() and outVectors.is_contiguous()):
             raise ValueError("blocks of vectors must be contiguous (row-major)")
-        if inVectors.shape[0] != self.info.columns or outVectors.shape[0] != self.info.rows:
+        if inVectors.shape[0] != self._columns or outVectors.shape[0] != self._rows:
             raise ValueError("vector sizes do not match the matrix")
         _check(lib.tnlhip_spmv_multi(self._h, int(inVectors.shape[1]), _ptr(inVectors), _ptr(outVectors),
                                      float(matrixMultiplicator), float(outVectorMultiplicator), int(firstRow),
