@@ -218,7 +218,7 @@ int tnlhip_matrix_get_storage( tnlhip_matrix A, double* values, int32_t* columns
 int tnlhip_matrix_get_diagonal( tnlhip_matrix A, void* diagonal, void* stream );
 
 /* Overrides a kernel parameter chosen at construction (FP32 / BF16 ChunkedEllpack and FP32
- * SlicedEllpack start with "xcd_remap" 1; Ellpack and FP64 / BF16 SlicedEllpack with "pair_rows" 1, "blocks_per_cu"
+ * SlicedEllpack start with "xcd_remap" 1; for rows of at most 8 slots on average Ellpack and FP64 / BF16 SlicedEllpack with "pair_rows" 1, "blocks_per_cu"
  * 32 and "xcd_remap" 1, but FP64 SlicedEllpack beyond 1500000 rows with "xcd_remap" 0 and FP32 Ellpack beyond
  * 3000000 rows with "xcd_remap" 3 and "pair_rows" 0; every other
  * matrix with "xcd_remap" 0, "pair_rows" 0, "blocks_per_cu" 16): "lanes_per_row" (CSR light / hybrid /

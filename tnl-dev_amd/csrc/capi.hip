@@ -164,8 +164,21 @@ tnlhip_matrix_s* buildFromSegments( int format, int dtype, int32_t rows, int32_t
    //                       order 17.9 33.1 70.8 53.8
    //   Ellpack FP32        the same 16.8 28.8 50.3 41.5 and 13.7 23.2 51.3 38.3 (taken up to 3 million rows)
    //   Ellpack BF16        one row, plain order 14.0 35.5 83.0 60.2; two rows, XCD order 11.4 19.4 41.5 32.6
+   // Rows of more than 8 slots on average keep the shapes they had (one row per lane; BF16 SlicedEllpack on lognormal
+   // rows of 17 entries 125 us, two rows per lane 211).
    const bool sliced = format == TNLHIP_SLICED_ELLPACK;
-   if( ( sliced && dtype != TNLHIP_F32 ) || format == TNLHIP_ELLPACK ) {
+   const bool shortRows = M->meta.allocated <= 8 * (int64_t) rows;
+   if( ! shortRows ) {
+      if( sliced && dtype != TNLHIP_F64 )
+         M->xcdRemap = 1;
+      if( format == TNLHIP_ELLPACK && dtype != TNLHIP_BF16 )
+         M->xcdRemap = 3;
+      if( ( format == TNLHIP_ELLPACK && dtype != TNLHIP_BF16 ) || ( sliced && dtype == TNLHIP_F64 ) )
+         M->blocksPerCu = 32;
+      if( sliced && dtype == TNLHIP_F64 )
+         M->pairRows = 1;
+   }
+   else if( ( sliced && dtype != TNLHIP_F32 ) || format == TNLHIP_ELLPACK ) {
       M->blocksPerCu = 32;
       M->pairRows = 1;
       M->xcdRemap = 1;

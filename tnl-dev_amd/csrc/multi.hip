@@ -430,6 +430,8 @@ bool launchShort( const Matrix& M, int32_t k, const Y* X, Y* Yv, double alpha, d
    const int64_t rows = (int64_t) last - first;
    if( wide && ( sizeof( Y ) != 8 || L < 4 || rows * L / kWave < kMultiManyTiles ) )
       return false;
+   if( rows < 200000 )  // FP32 k = 7, CSR: 132000 rows 9.5 / 10.5, 262000 rows 16.5 / 13.6
+      return false;
    if( KP == 4 && ( sizeof( Y ) != 8 || kindOf( M.format ) == KIND_CSR || rows < 1000000 ) )
       return false;
    if constexpr( L >= 2 ) {

@@ -207,9 +207,7 @@ __device__ __forceinline__ void csrScalarStagedRows( const int32_t* __restrict__
    const int32_t re = mine ? off[ r + 1 ] : 0;
    const int32_t b = __shfl( rb, 0, kWave );
    const int32_t size = __shfl( re, max( used, 1 ) - 1, kWave ) - b;
-   int32_t c[ kStageLoads ];
-   V v[ kStageLoads ];
-   auto loadRound = [ & ]( int32_t e0 ) {
+   auto loadRound = [ & ]( int32_t e0, int32_t ( &c )[ kStageLoads ], V ( &v )[ kStageLoads ] ) {
 #pragma unroll
       for( int k = 0; k < kStageLoads; k++ ) {
          c[ k ] = -1;
@@ -221,9 +219,11 @@ __device__ __forceinline__ void csrScalarStagedRows( const int32_t* __restrict__
          }
       }
    };
+   int32_t c0[ kStageLoads ];  // a fused product's first round, loaded before begin()
+   V v0[ kStageLoads ];
    if constexpr( ! Keep::kPlain ) {
       if( size > 0 )
-         loadRound( 0 );
+         loadRound( 0, c0, v0 );
       if( ! keep.begin() || ! any )
          return;
    }
@@ -240,8 +240,17 @@ __device__ __forceinline__ void csrScalarStagedRows( const int32_t* __restrict__
          const int32_t e0 = q * kStageLoads * kWave;
          if( e0 >= size )  // uniform over the wave
             break;
+         int32_t c[ kStageLoads ];
+         V v[ kStageLoads ];
          if( Keep::kPlain || q > 0 )
-            loadRound( e0 );
+            loadRound( e0, c, v );
+         else {
+#pragma unroll
+            for( int k = 0; k < kStageLoads; k++ ) {
+               c[ k ] = c0[ k ];
+               v[ k ] = v0[ k ];
+            }
+         }
          Y xv[ kStageLoads ];
 #pragma unroll
          for( int k = 0; k < kStageLoads; k++ )
