@@ -286,6 +286,24 @@ def test_polynomial_start_in_the_product_of_every_format(tnl, dev, fmt, dt, degr
     np.testing.assert_allclose(got[3][:8], want[3][:8], rtol=1e-9 if dt == "f64" else 1e-3)
 
 
+def test_polynomial_over_a_striped_plan(tnl, dev):
+    # a striped plan forms z_0 in a pass of its own; its row sums differ from the plain product's by
+    # their order alone
+    rp, c, v = W.convection_diffusion_3d(9, 10.0)
+    b = t(W.uniform_vector(len(rp) - 1, 4), dev)
+    h = []
+    for stripes in (0, 4):
+        A = tnl.SparseMatrix.from_csr(rp, c, v, format="CSRAdaptive", dtype="f64")
+        A.set_param("column_stripes", stripes)
+        s = tnl.getLinearSolver("gmres")
+        s.setMatrix(A)
+        s.setup(convergence_residue=1e-9, max_iterations=200, preconditioner=3, restarting_min=10, restarting_max=10)
+        assert s.solve(b, torch.zeros_like(b))
+        h.append(s.getResidualHistory())
+    assert abs(len(h[0]) - len(h[1])) <= 1
+    np.testing.assert_allclose(h[0][:8], h[1][:8], rtol=1e-9)
+
+
 @pytest.mark.parametrize("method", ["cg", "bicgstab"])
 @pytest.mark.parametrize("most", [0, 1, 2, 11, 12, 13, 29])
 def test_iteration_limits_of_fused_solves(tnl, dev, method, most):

@@ -139,7 +139,9 @@ void spmvMultiLaunch( const Matrix& A, int32_t k, const void* X, void* Y, double
 // as above (general real-valued P only; znew aliases neither z nor rhs)
 void spmvJacobiStepGated( const Matrix& P, const void* z, void* znew, const void* rhs, const void* diag,
                           const int32_t* gate, int gateMode, hipStream_t stream );
-// y = A x and quotient = y / diag over all rows in one product, gated as above (general real-valued A)
+// y = A x and quotient = y / diag over all rows in one product, gated as above, for the matrices that
+// quotientProduct names (general real-valued ones without a striped plan)
+bool quotientProduct( const Matrix& A );
 void spmvQuotientGated( const Matrix& A, const void* x, void* y, void* quotient, const void* diag,
                         const int32_t* gate, int gateMode, hipStream_t stream );
 // SymmetricMatrix product (symmetric.hip), used by spmvLaunchGated for symmetric matrices

@@ -400,17 +400,17 @@ void precSolve( SolverImpl& S, const void* in, void* out, Gate gate )
 void matvec( SolverImpl& S, const void* x, void* y, Gate gate )
 {
    if( S.params.preconditioner == 3 ) {
-      // A x into the polynomial's input vector, then the polynomial into y (no copy); a general matrix's
-      // product writes z_0 = D^-1 A x beside it
-      const bool general = ! S.A->symmetric;
+      // A x into the polynomial's input vector, then the polynomial into y (no copy); most products write
+      // z_0 = D^-1 A x beside it
+      const bool quotient = quotientProduct( *S.A );
       auto apply = [ & ]( auto* tag ) {
          using T = std::remove_pointer_t< decltype( tag ) >;
-         if( general )
+         if( quotient )
             spmvQuotientGated( *S.A, x, S.polyVecs.ptr, polyBuffer< T >( S, y, 0 ), S.diag.ptr, gate.flags, gate.mode,
                                S.stream );
          else
             spmvLaunchGated( *S.A, x, S.polyVecs.ptr, 1.0, 0.0, nullptr, gate.flags, gate.mode, S.stream );
-         polyApplyTyped< T >( S, S.polyVecs.ptr, y, gate, general );
+         polyApplyTyped< T >( S, S.polyVecs.ptr, y, gate, quotient );
       };
       if( S.vdtype == TNLHIP_F64 )
          apply( (double*) nullptr );

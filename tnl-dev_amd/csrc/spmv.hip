@@ -11,17 +11,13 @@ namespace {
 template< typename V, typename A, typename Y >
 void launchTyped( const Matrix& M, const Y* x, Y* y, double alpha, double beta, int32_t first, int32_t last,
                   const Y* diag, const int32_t* gate, int gateMode, hipStream_t st, const Y* rhs = nullptr,
-                  const Y* prev = nullptr, Y* quotient = nullptr )
+                  const Y* prev = nullptr )
 {
    Keeper< A, Y > keep{ y, (A) alpha, (A) beta, diag, 0, gate, gate ? gateMode : 0 };
    if( rhs ) {
       keep.mode = 5;
       keep.rhs = rhs;
       keep.prev = prev;
-   }
-   else if( quotient ) {
-      keep.mode = 6;
-      keep.y2 = quotient;
    }
    else if( diag )
       keep.mode = 4;
@@ -91,17 +87,24 @@ void spmvJacobiStepGated( const Matrix& P, const void* z, void* znew, const void
    }
 }
 
+bool quotientProduct( const Matrix& A )
+{
+   return A.dtype != TNLHIP_BINARY && ! A.symmetric && ! A.stripes;
+}
+
 void spmvQuotientGated( const Matrix& A, const void* x, void* y, void* quotient, const void* diag,
                         const int32_t* gate, int gateMode, hipStream_t stream )
 {
-   if( A.dtype == TNLHIP_BINARY || A.symmetric )
-      throw Error( TNLHIP_ERROR_UNSUPPORTED, "products with a quotient take general real-valued matrices" );
+   if( ! quotientProduct( A ) )
+      throw Error( TNLHIP_ERROR_UNSUPPORTED, "products with a quotient take general real-valued matrices without a "
+                                             "striped plan" );
    TNLHIP_REQUIRE( y != quotient, "the product and its quotient are two vectors" );
    auto launch = [ & ]( auto* tagV, auto* tagY ) {
       using V = std::remove_pointer_t< decltype( tagV ) >;
       using Y = std::remove_pointer_t< decltype( tagY ) >;
-      launchTyped< V, Y, Y >( A, (const Y*) x, (Y*) y, 1.0, 0.0, 0, A.rows, (const Y*) diag, gate, gateMode, stream,
-                              nullptr, nullptr, (Y*) quotient );
+      const QuotientKeeper< Y, Y > keep{ { (Y*) y, (Y) 1, (Y) 0, (const Y*) diag, 0, gate, gate ? gateMode : 0 },
+                                         (Y*) quotient };
+      launchProduct< V, Y, Y >( A, (const Y*) x, keep, 0, A.rows, stream );
    };
    switch( A.dtype ) {
       case TNLHIP_F64: launch( (double*) nullptr, (double*) nullptr ); break;

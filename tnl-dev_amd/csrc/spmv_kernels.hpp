@@ -21,8 +21,9 @@
 #include "spmv.hpp"
 #include "rowdist.hpp"
 
-namespace tnlhip {
+#include <type_traits>
 
+namespace tnlhip {
 
 template< bool EXACT, typename A >
 __device__ __forceinline__ A madd( A acc, A a, A b )
@@ -907,7 +908,7 @@ unsigned launchProduct( const Matrix& M, const Y* x, Keep keep, int32_t first, i
       return 0;
    }
    if( M.stripes && kindOf( M.format ) == KIND_CSR ) {
-      if constexpr( Keep::kPlain )
+      if constexpr( std::is_same_v< Keep, Keeper< A, Y > > )
          stripeLaunch< V, A, Y >( M, x, keep, first, last, st );
       return 0;
    }
