@@ -415,3 +415,28 @@ def test_binary_products(tnl, dev, fmt):
     s.setMatrix(A)
     with pytest.raises(tnl.TnlHipError, match="binary"):
         s.solve(torch.zeros(500, dtype=torch.float32, device=dev), torch.zeros(500, dtype=torch.float32, device=dev))
+
+
+@pytest.mark.parametrize("fmt", ["SlicedEllpack", "Ellpack", "ChunkedEllpack"])
+@pytest.mark.parametrize("most", [8, 9, 16, 31, 32, 33, 41])
+def test_rows_around_whole_chunks_of_slots(tnl, dev, fmt, most):
+    # two rows per lane, row lengths that end at, before and after chunks of 8 slots, and mean lengths on both
+    # sides of the 32 slots from which SlicedEllpack re-reads the last slot instead of leaving slots out
+    rng = np.random.default_rng(most)
+    n = 2113
+    per = np.where(rng.random(n) < 0.9, most, rng.integers(0, most + 1, n))
+    rp = np.zeros(n + 1, np.int32)
+    np.cumsum(per, out=rp[1:])
+    c = np.concatenate([np.sort(rng.choice(n, k, replace=False)) for k in per]).astype(np.int32)
+    v = rng.uniform(-1, 1, len(c))
+    x = rng.uniform(-1, 1, n)
+    want = O.Segments("CSR", per.astype(np.int32)).spmv(v, c, x)
+    A = tnl.SparseMatrix.from_csr(rp, c, v, format=fmt, dtype="f64")
+    A.set_param("pair_rows", 1)
+    y = torch.full((n,), np.nan, dtype=torch.float64, device=dev)
+    A.vectorProduct(torch.tensor(x, device=dev), y)
+    if fmt == "ChunkedEllpack":  # sums of up to 41 products in another order
+        mag = np.bincount(np.repeat(np.arange(n), per), weights=np.abs(v * x[c]), minlength=n)
+        assert np.all(np.abs(y.cpu().numpy() - want) <= 41 * 2.0 ** -53 * 2 * mag)
+    else:
+        assert np.array_equal(y.cpu().numpy(), want)

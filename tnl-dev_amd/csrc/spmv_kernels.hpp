@@ -60,9 +60,9 @@ __device__ __forceinline__ bf16 ldnt( const bf16* p )
 // whole waves or lane pairs take) instead of re-reading the last slot: from `least` value bytes on.  The
 // branches keep narrow loads from being issued together.  us, re-read / left out, at 160^3 and 2000^2:
 // staged CSR FP64 76.9 61.6 / 74.9 53.8, FP32 56.9 43.0 / 57.4 40.2, BF16 52.5 40.0 / 69.5 48.9;
-// CSRAdaptive FP64 79.9 57.7 / 78.0 56.5, FP32 61.9 43.7 / 60.9 42.1, BF16 56.9 39.4 / 71.2 51.3;
-// ChunkedEllpack FP64 71.1 59.6 / 68.5 54.0, FP32 46.3 38.4 / 50.3 38.4; BiEllpack FP64 77.1 68.7 / 72.1 56.3,
-// FP32 48.9 47.1 / 46.5 41.3, BF16 42.3 42.6 / 58.6 49.1.
+// CSRAdaptive FP64 79.9 57.7 / 78.0 56.5, FP32 61.9 43.7 / 60.9 42.1 but on 40-entry rows 113 / 129, BF16
+// 56.9 39.4 / 71.2 51.3; ChunkedEllpack FP64 71.1 59.6 / 68.5 54.0, FP32 46.3 38.4 / 50.3 38.4; BiEllpack FP64
+// 77.1 68.7 / 72.1 56.3, FP32 48.9 47.1 / 46.5 41.3, BF16 42.3 42.6 / 58.6 49.1.
 // An operand that is formed where it is gathered keeps the straight line (64^3 CG, SlicedEllpack: 14.8 us per iteration
 // against 18.0).
 template< typename V, typename Keep, int least >
@@ -207,7 +207,8 @@ __device__ __forceinline__ void csrScalarStagedRows( const int32_t* __restrict__
    const int32_t rb = mine ? off[ r ] : 0;
    const int32_t re = mine ? off[ r + 1 ] : 0;
    const int32_t b = __shfl( rb, 0, kWave );
-   const int32_t size = __shfl( re, max( used, 1 ) - 1, kWave ) - b;
+   // (a plain product's wave has rows)
+   const int32_t size = __shfl( re, Keep::kPlain ? used - 1 : max( used, 1 ) - 1, kWave ) - b;
    auto loadRound = [ & ]( int32_t e0, int32_t ( &c )[ kStageLoads ], V ( &v )[ kStageLoads ] ) {
 #pragma unroll
       for( int k = 0; k < kStageLoads; k++ ) {
@@ -359,7 +360,7 @@ __global__ __launch_bounds__( 256 ) void csrAdaptiveKernel( int32_t nblocks, con
          for( int k = 0; k < kStageLoads; k++ ) {
             c[ k ] = -1;
             v[ k ] = V( 0.0f );
-            if( ! kSkipSlots< V, Keep, 4 > || e0 + k * kWave < size ) {  // uniform over the wave
+            if( ! kSkipSlots< V, Keep, 8 > || e0 + k * kWave < size ) {  // uniform over the wave
                const int32_t e = min( e0 + lane + k * kWave, size - 1 );
                c[ k ] = ldnt( col + b + e );
                v[ k ] = ldnt( val + b + e );
@@ -369,7 +370,7 @@ __global__ __launch_bounds__( 256 ) void csrAdaptiveKernel( int32_t nblocks, con
 #pragma unroll
          for( int k = 0; k < kStageLoads; k++ ) {
             xv[ k ] = Y( 0 );
-            if( ! kSkipSlots< V, Keep, 4 > || e0 + k * kWave < size )
+            if( ! kSkipSlots< V, Keep, 8 > || e0 + k * kWave < size )
                xv[ k ] = keep.at( x, c[ k ] < 0 ? 0 : c[ k ] );
          }
 #pragma unroll
@@ -491,11 +492,15 @@ __device__ __forceinline__ int2 ldnt2( const int32_t* p )
    return make_int2( (int32_t) ( v & 0xffffffff ), (int32_t) ( v >> 32 ) );
 }
 
-// One or two (PAIR) rows per lane.  A chunk's slots beyond the row's width are neither loaded nor
-// gathered (whole waves skip them): re-reading the last slot instead, as a lane pair did before, cost
-// a 5-wide row 3 of 8 loads (FP64 SlicedEllpack 160^3 77.1 -> 69.6 us, 128^3 41.2 -> 37.0, 2000^2 69.9 ->
-// 51.6).  Slot index of row r at local index l: base( r ) + step * l.
-template< bool PAIR, typename V, typename A, typename Y, typename Keep, typename Slots >
+// One or two (PAIR) rows per lane.  Slot index of row r at local index l: base( r ) + step * l.
+// With SKIP a lane pair neither loads nor gathers a chunk's slots beyond the row's width (whole waves skip
+// them): re-reading the last slot instead costs a 5-wide row 3 of 8 loads (FP64 SlicedEllpack 160^3
+// 77.1 -> 69.6 us, 128^3 41.2 -> 37.0, 2000^2 69.9 -> 51.6).  The branches cost registers (72 -> 96 in FP64, 7
+// -> 5 waves per SIMD), so rows of more than kSkipSlotsUpTo slots on average, whose chunks are mostly full,
+// re-read (FP64 SlicedEllpack, re-read / left out: 27 slots 49.5 / 45.6 us, 30 75.6 / 76.3, 34 103.3 / 108.8,
+// 73 173.9 / 182.8).  One row per lane re-reads x[ 0 ] for such slots, and its last row the last slot.
+constexpr int kSkipSlotsUpTo = 32;
+template< bool PAIR, bool SKIP, typename V, typename A, typename Y, typename Keep, typename Slots >
 __device__ __forceinline__ void paddedRows( const Slots& slots, const int32_t* __restrict__ col,
                                             const V* __restrict__ val, const Y* __restrict__ x, Keep& keep,
                                             int32_t first, RowSeq seq )
@@ -554,7 +559,7 @@ __device__ __forceinline__ void paddedRows( const Slots& slots, const int32_t* _
    }
    // a fused product's first chunk is loaded before begin()
    constexpr bool kAhead = PAIR && ! Keep::kPlain;
-   constexpr bool kSkip = kSkipSlots< V, Keep, 1 >;
+   constexpr bool kSkip = SKIP && kSkipSlots< V, Keep, 1 >;
    int2 c[ kChunk ];
    typename Pair< V >::T v[ kChunk ];
    auto loadChunk = [ & ]( int64_t b, int32_t l0, int32_t width, int64_t step ) {
@@ -584,7 +589,32 @@ __device__ __forceinline__ void paddedRows( const Slots& slots, const int32_t* _
       const int64_t step = slots.step();
       A s0 = 0, s1 = 0;
       for( int32_t l0 = 0; l0 < width; l0 += kChunk ) {
-         if constexpr( PAIR ) {
+         if constexpr( PAIR && ! kSkip && ! kAhead ) {
+            int2 c[ kChunk ];
+            typename Pair< V >::T v[ kChunk ];
+#pragma unroll
+            for( int j = 0; j < kChunk; j++ ) {
+               const int64_t g = b + step * min( l0 + j, width - 1 );
+               c[ j ] = ldnt2( col + g );
+               v[ j ] = ldnt2( val + g );
+            }
+            Y x0[ kChunk ], x1[ kChunk ];
+#pragma unroll
+            for( int j = 0; j < kChunk; j++ ) {
+               x0[ j ] = keep.at( x, c[ j ].x < 0 ? 0 : c[ j ].x );
+               x1[ j ] = keep.at( x, c[ j ].y < 0 ? 0 : c[ j ].y );
+            }
+#pragma unroll
+            for( int j = 0; j < kChunk; j++ ) {
+               V a, bb;
+               split( v[ j ], a, bb );
+               if( l0 + j < width && c[ j ].x >= 0 )
+                  s0 = mulAddExact( s0, toCompute( a, A() ), (A) x0[ j ] );
+               if( l0 + j < width && c[ j ].y >= 0 )
+                  s1 = mulAddExact( s1, toCompute( bb, A() ), (A) x1[ j ] );
+            }
+         }
+         else if constexpr( PAIR ) {
             if( ! kAhead || ! ahead )
                loadChunk( b, l0, width, step );
             ahead = false;
@@ -665,11 +695,11 @@ __global__ __launch_bounds__( 256 ) void ellpackKernel( EllpackSlots slots, cons
    else if( ! openKeeper( keep ) )
       return;
    const int64_t base = PAIR ? ( first & ~1 ) : first;
-   paddedRows< PAIR, V, A >( slots, col, val, x, keep, first, rowSequence< PAIR ? 2 : 1 >( base, last, rowsPerBlock, dist ) );
+   paddedRows< PAIR, true, V, A >( slots, col, val, x, keep, first, rowSequence< PAIR ? 2 : 1 >( base, last, rowsPerBlock, dist ) );
    keep.finish();
 }
 
-template< bool PAIR, typename V, typename A, typename Y, typename Keep >
+template< bool PAIR, bool SKIP, typename V, typename A, typename Y, typename Keep >
 __global__ __launch_bounds__( 256 ) void slicedKernel( SlicedSlots slots, const int32_t* __restrict__ col,
                                                        const V* __restrict__ val, const Y* __restrict__ x,
                                                        Keep keep, int32_t first, int32_t last,
@@ -680,7 +710,7 @@ __global__ __launch_bounds__( 256 ) void slicedKernel( SlicedSlots slots, const 
    else if( ! openKeeper( keep ) )
       return;
    const int64_t base = PAIR ? ( first & ~1 ) : first;
-   paddedRows< PAIR, V, A >( slots, col, val, x, keep, first, rowSequence< PAIR ? 2 : 1 >( base, last, rowsPerBlock, dist ) );
+   paddedRows< PAIR, SKIP, V, A >( slots, col, val, x, keep, first, rowSequence< PAIR ? 2 : 1 >( base, last, rowsPerBlock, dist ) );
    keep.finish();
 }
 
@@ -715,29 +745,57 @@ __global__ __launch_bounds__( 256 ) void chunkedKernel( int32_t nslices, const i
       A p = 0;
       for( int32_t k0 = 0; k0 < s.y; k0 += kChunk ) {
          int32_t c[ kChunk ];
-         V v[ kChunk ];
+         if constexpr( kSkipSlots< V, Keep, 8 > ) {
+            // `full`: every slot of the round exists, and its loads go out without a branch between them (FP64,
+            // lognormal rows of 6 entries on average, 1 million of them: 307 us with the branches in every round, 264
+            // with re-read slots, 240; 150^3 Laplacian 58.3 / 59.4 / 56.5)
+            auto round = [ & ]( auto full ) {
+               constexpr bool kFull = decltype( full )::value;
+               V v[ kChunk ];
+               Y xv[ kChunk ];
 #pragma unroll
-         for( int j = 0; j < kChunk; j++ ) {
-            c[ j ] = -1;
-            v[ j ] = V( 0.0f );
-            if( ! kSkipSlots< V, Keep, 8 > || k0 + j < s.y ) {  // uniform over the workgroup
-               const int32_t l = kSkipSlots< V, Keep, 8 > ? k0 + j : min( k0 + j, s.y - 1 );
-               const int64_t g = (int64_t) s.w + t + (int64_t) kChunksInSlice * l;
+               for( int j = 0; j < kChunk; j++ ) {
+                  c[ j ] = -1;
+                  v[ j ] = V( 0.0f );
+                  if( kFull || k0 + j < s.y ) {  // uniform over the workgroup
+                     const int64_t g = (int64_t) s.w + t + (int64_t) kChunksInSlice * ( k0 + j );
+                     c[ j ] = ldnt( col + g );
+                     v[ j ] = ldnt( val + g );
+                  }
+               }
+#pragma unroll
+               for( int j = 0; j < kChunk; j++ ) {
+                  xv[ j ] = Y( 0 );
+                  if( kFull || k0 + j < s.y )
+                     xv[ j ] = keep.at( x, c[ j ] < 0 ? 0 : c[ j ] );
+               }
+#pragma unroll
+               for( int j = 0; j < kChunk; j++ )
+                  if( c[ j ] >= 0 )
+                     p += toCompute( v[ j ], A() ) * (A) xv[ j ];
+            };
+            if( k0 + kChunk <= s.y )
+               round( std::true_type() );
+            else
+               round( std::false_type() );
+         }
+         else {
+            V v[ kChunk ];
+#pragma unroll
+            for( int j = 0; j < kChunk; j++ ) {
+               const int64_t g = (int64_t) s.w + t + (int64_t) kChunksInSlice * min( k0 + j, s.y - 1 );
                c[ j ] = ldnt( col + g );
                v[ j ] = ldnt( val + g );
             }
-         }
-         Y xv[ kChunk ];
+            Y xv[ kChunk ];
 #pragma unroll
-         for( int j = 0; j < kChunk; j++ ) {
-            xv[ j ] = Y( 0 );
-            if( ! kSkipSlots< V, Keep, 8 > || k0 + j < s.y )
+            for( int j = 0; j < kChunk; j++ )
                xv[ j ] = keep.at( x, c[ j ] < 0 ? 0 : c[ j ] );
-         }
 #pragma unroll
-         for( int j = 0; j < kChunk; j++ )
-            if( ( kSkipSlots< V, Keep, 8 > || k0 + j < s.y ) && c[ j ] >= 0 )
-               p += toCompute( v[ j ], A() ) * (A) xv[ j ];
+            for( int j = 0; j < kChunk; j++ )
+               if( k0 + j < s.y && c[ j ] >= 0 )
+                  p += toCompute( v[ j ], A() ) * (A) xv[ j ];
+         }
          // the last slot read is padding: so is the rest of this lane's chunk
          if( stopAtPadding && __all( c[ kChunk - 1 ] < 0 ) )
             break;  // wave-uniform; the loop holds no barrier
@@ -1006,11 +1064,19 @@ unsigned launchProduct( const Matrix& M, const Y* x, Keep keep, int32_t first, i
                     dist );
          }
          else {
-            if( pair )
-               run( slicedKernel< true, V, A, Y, Keep >, grid, ss, col, val, x, keep, first, last, (int32_t) per,
+            // (a fused product's rows take the registers either way)
+            bool skip = true;
+            if constexpr( Keep::kPlain ) {
+               skip = M.meta.allocated <= (int64_t) kSkipSlotsUpTo * M.rows;
+               if( pair && ! skip )
+                  run( slicedKernel< true, false, V, A, Y, Keep >, grid, ss, col, val, x, keep, first, last, (int32_t) per,
+                       dist );
+            }
+            if( pair && skip )
+               run( slicedKernel< true, true, V, A, Y, Keep >, grid, ss, col, val, x, keep, first, last, (int32_t) per,
                     dist );
-            else
-               run( slicedKernel< false, V, A, Y, Keep >, grid, ss, col, val, x, keep, first, last, (int32_t) per,
+            if( ! pair )
+               run( slicedKernel< false, true, V, A, Y, Keep >, grid, ss, col, val, x, keep, first, last, (int32_t) per,
                     dist );
          }
          break;
