@@ -1,6 +1,7 @@
 """Reductions, BLAS-1 and the Krylov solvers on the GPU through the C ABI, against the oracle
 (single-thread TNL semantics, pinned to TNL's own residual histories) and the mathematics."""
 import os
+import time
 import numpy as np
 import pytest
 import torch
@@ -233,6 +234,54 @@ def test_fused_iterations_follow_the_oracle(tnl, dev, fmt, n):
                 continue
             assert abs(s.getIterations() - ref["iterations"]) <= 1
             np.testing.assert_allclose(xd.cpu().numpy(), ref["x"], rtol=0, atol=1e-8 * np.abs(ref["x"]).max())
+
+
+def _arrow(n, m):
+    """Tridiagonal with m more entries in row 0 and column 0, symmetric and diagonally dominant."""
+    i = np.arange(n)
+    e = np.sort(np.random.default_rng(1).choice(np.arange(2, n), m, replace=False))
+    r = np.concatenate([i[1:], i, i[:-1], np.zeros(m, int), e])
+    c = np.concatenate([i[1:] - 1, i, i[:-1] + 1, e, np.zeros(m, int)])
+    d = np.full(n, 4.0)
+    d[0] += 1e-3 * m
+    v = np.concatenate([np.full(n - 1, -1.0), d, np.full(n - 1, -1.0), np.full(2 * m, 1e-3)])
+    o = np.lexsort((c, r))
+    rp = np.zeros(n + 1, np.int32)
+    np.cumsum(np.bincount(r, minlength=n), out=rp[1:])
+    return rp, c[o].astype(np.int32), v[o]
+
+
+@pytest.mark.parametrize("method,products", [("cg", 1), ("bicgstab", 2)])
+def test_one_long_row_among_short_ones_keeps_its_kernel(tnl, dev, method, products):
+    """A solve over CSRAdaptive splits a long row over a workgroup as its product does: an iteration costs about
+    two products each (its vector passes included); walked by one lane the row alone costs about 60."""
+    rp, c, v = _arrow(200000, 20000)
+    n = len(rp) - 1
+    A = tnl.SparseMatrix.from_csr(rp, c, v, format="CSRAdaptive", dtype="f64")
+    b = t(W.uniform_vector(n, 2), dev)
+    y = torch.zeros_like(b)
+    e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    A.vectorProduct(b, y)
+    e0.record()
+    for _ in range(10):
+        A.vectorProduct(b, y)
+    e1.record()
+    e1.synchronize()
+    product = e0.elapsed_time(e1) / 10
+    s = tnl.getLinearSolver(method)
+    s.setMatrix(A)
+    s.setup(convergence_residue=1e-300, max_iterations=8)
+    best = 1e9
+    for _ in range(3):
+        x = torch.zeros_like(b)
+        torch.cuda.synchronize()
+        start = time.perf_counter()
+        s.solve(b, x)
+        best = min(best, 1e3 * (time.perf_counter() - start))
+    assert best / s.getIterations() < 12 * products * product, (best, product)
+    ref = O.solve(method, rp, c, v, b.cpu().numpy(), convergence_residue=1e-300, max_iterations=8)
+    # sums of 200000 and of 20000 products in another order: 1e-13 each, amplified by the steps
+    np.testing.assert_allclose(s.getResidualHistory()[:6], ref["history"][:6], rtol=1e-8)
 
 
 @pytest.mark.parametrize("m", [1, 700, 110000])  # the last beyond the rows whose operand the product forms

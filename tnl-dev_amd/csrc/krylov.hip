@@ -33,9 +33,16 @@ struct FusedKeeper
 
 }  // namespace
 
-int fusedGrid( const Matrix& A )
+int fusedGrid( const Matrix& A, bool twoProducts )
 {
    if( A.symmetric || ( A.dtype != TNLHIP_F64 && A.dtype != TNLHIP_F32 ) || A.meta.allocated == 0 )
+      return 0;
+   // With 32 or 64 lanes a row one lane in so many adds up a wave's dots, behind the row's sum; launches saved pay for
+   // it only where they count.  us per iteration, separate passes / fused, 27-point box, CSRLight (32 lanes) FP64: CG
+   // 40^3 25.5 / 24.4, 52^3 34.4 / 34.5, 90^3 86.1 / 95.5; BiCGStab 52^3 70.6 / 58.5, 90^3 168 / 172; CSRVector (64
+   // lanes) CG 52^3 47.3 / 49.8, 90^3 176 / 197, BiCGStab 500000 rows of 40 entries 365 / 366, 90^3 343 / 364.
+   if( kindOf( A.format ) == KIND_CSR && A.format != TNLHIP_CSR_ADAPTIVE && lanesPerRow( A ) >= 32 &&
+       A.rows > ( twoProducts ? 500000 : 100000 ) )
       return 0;
    unsigned grid;
    if( A.dtype == TNLHIP_F64 )
@@ -57,10 +64,16 @@ int fusedGrid( const Matrix& A )
 // product / in a pass of its own: CG 2D 256^2 11.2 / 13.3 (SlicedEllpack), 11.9 / 13.2 (CSRScalar);
 // 64^3 14.9 / 16.5, 18.9 / 18.8; 80^3 26.4 / 26.8, 30.6 / 30.2; 100^3 42.3 / 41.1, 48.2 / 42.3.
 // BiCGStab (three vectors) 256^2 20.0 / 23.0, 20.6 / 22.3; 64^3 28.5 / 29.2, 34.9 / 35.3; 80^3
-// 49.8 / 46.9, 62.7 / 53.1.  So it pays while the launches count: up to 300000 short rows.
+// 49.8 / 46.9, 62.7 / 53.1.  So it pays while the launches count: up to 300000 short rows, in CSR only where no
+// lane walks a row (200000 rows of 3 with one of 20000, CG: 5645 / 4739) and no lane group shares one (65^3, 8 and 64
+// lanes, CG: 34.5 / 32.3 and 84.6 / 76.7).
 bool fuseOperand( const Matrix& A )
 {
-   return A.meta.allocated <= (int64_t) kShortRow * A.rows && A.rows <= 300000;
+   if( A.meta.allocated > (int64_t) kShortRow * A.rows || A.rows > 300000 )
+      return false;
+   if( kindOf( A.format ) != KIND_CSR )
+      return true;
+   return A.dtype == TNLHIP_F64 ? stagedThroughout< double >( A ) : stagedThroughout< float >( A );
 }
 
 template< typename T, typename Op >

@@ -717,8 +717,8 @@ constexpr int kMaxFusedPartials = 8192;
 
 // The grid, hence the number of partials per sum, of the fused products with A; 0 when A takes the
 // separate passes (symmetric, binary and BF16 matrices, striped plans, nothing stored, more than
-// kMaxFusedPartials workgroups).
-int fusedGrid( const Matrix& A );
+// kMaxFusedPartials workgroups, many rows of 32 or 64 lanes).  twoProducts: an iteration has two of them (BiCGStab).
+int fusedGrid( const Matrix& A, bool twoProducts );
 
 // Whether forming the operand where it is gathered pays for A.
 bool fuseOperand( const Matrix& A );

@@ -941,7 +941,7 @@ void solveCG( SolverImpl& S, const void* b, void* xv )
    const T* diag = S.params.preconditioner == 1 ? (const T*) S.diag.ptr : nullptr;
    const Gate always{ nullptr, 0 }, running{ S.state.ptr->flags, 1 };
    const Stop stop = S.stopRule();
-   if( const int grid = fusedGrid( *S.A ) ) {
+   if( const int grid = fusedGrid( *S.A, false ) ) {
       solveCGFused< T >( S, b, x, grid );
       return;
    }
@@ -1344,7 +1344,7 @@ void solveBiCGStab( SolverImpl& S, const void* b, void* xv )
    const Gate always{ nullptr, 0 }, running{ S.state.ptr->flags, 1 }, restart{ S.state.ptr->flags, 2 };
    const Stop stop = S.stopRule();
    const double eps = std::numeric_limits< T >::epsilon();
-   const int fused = ! exact && S.params.preconditioner <= 1 ? fusedGrid( *S.A ) : 0;
+   const int fused = ! exact && S.params.preconditioner <= 1 ? fusedGrid( *S.A, true ) : 0;
    if( fused ) {
       solveBiCGStabFused< T >( S, b, x, fused );
       return;

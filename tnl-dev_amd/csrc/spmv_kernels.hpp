@@ -925,6 +925,22 @@ __global__ __launch_bounds__( 256 ) void zeroRowsKernel( Keep keep, int32_t firs
 
 // ------------------------------------------------------------------ launch
 
+// Lanes per row of the cooperative CSR kernel; 0 where the rows take the staged one
+inline int lanesPerRow( const Matrix& M )
+{
+   if( M.format == TNLHIP_CSR_SCALAR || ( ! M.lanesExplicit && M.meta.allocated <= (int64_t) kShortRow * M.rows ) )
+      return 0;
+   return M.format == TNLHIP_CSR_VECTOR && ! M.lanesExplicit ? kWave : M.lanes;
+}
+
+// Whether M's rows take the staged CSR kernel with every wave's elements in LDS, none walking its rows one lane each
+template< typename A >
+bool stagedThroughout( const Matrix& M )
+{
+   return kindOf( M.format ) == KIND_CSR && lanesPerRow( M ) == 0 && M.meta.allocated <= (int64_t) kShortRow * M.rows &&
+          M.waveMost <= kAdaptiveStreamBytesPerWave / (int) sizeof( A );
+}
+
 // Launches the row kernel of M's format over rows [first, last) and returns its grid, or with `dry`
 // only returns the grid; 0 when no row kernel runs (no rows, no columns, a striped plan, no storage).
 template< typename V, typename A, typename Y, typename Keep >
@@ -978,10 +994,11 @@ unsigned launchProduct( const Matrix& M, const Y* x, Keep keep, int32_t first, i
       case TNLHIP_CSR_LIGHT:
       case TNLHIP_CSR_HYBRID:
       case TNLHIP_CSR_ADAPTIVE: {
-         // (a fused product of short rows takes the staged kernel, which hides the fold)
-         const bool shortRows = M.meta.allocated <= (int64_t) kShortRow * M.rows;
+         // a fused product of short rows takes the staged kernel, which hides the fold, unless some of its waves would
+         // walk their rows (us per CG iteration with a row of 20000 elements among 200000 of 3: 5180 staged, 82 here; per BiCGStab
+         // iteration with 1 million lognormal rows of 6: 764, 177)
          if( M.format == TNLHIP_CSR_ADAPTIVE && first == 0 && last == M.rows && M.adaptiveBlocks > 0 &&
-             ( Keep::kPlain || ! shortRows ) ) {
+             ( Keep::kPlain || ! stagedThroughout< A >( M ) ) ) {
             constexpr int STREAM = kAdaptiveStreamBytesPerWave / sizeof( A );
             // y through L2 on request (STREAM blocks end rows anywhere in a cache line of y, so
             // non-temporal stores write some lines twice); non-temporal by default, which measured
@@ -999,11 +1016,11 @@ unsigned launchProduct( const Matrix& M, const Y* x, Keep keep, int32_t first, i
          // rows of at most kShortRow stored elements on average: most lanes of a cooperative row
          // group would idle (a wavefront per 7-element row uses 7 of 64), so unless lanes_per_row
          // was set the rows take CSRScalar's staged kernel (the Host result bit for bit)
-         if( ! M.lanesExplicit && shortRows ) {
+         const int G = lanesPerRow( M );
+         if( G == 0 ) {
             launchStaged();
             break;
          }
-         const int G = M.format == TNLHIP_CSR_VECTOR && ! M.lanesExplicit ? 64 : M.lanes;
          const int gpb = 256 / G;
          const unsigned grid = gridFor( rows, gpb );
          switch( G ) {
