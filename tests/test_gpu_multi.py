@@ -144,9 +144,10 @@ def test_block_product_unaligned_blocks_take_the_scalar_lanes(tnl, dev):
 @pytest.mark.parametrize("dt", ["f64", "f32"])
 @pytest.mark.parametrize("k", [3, 5, 7, 9, 12, 16, 17, 33, 64])
 def test_short_rows_equal_the_columns_one_by_one(tnl, dev, fmt, dt, k):
-    # 65 x 67 x 61 rows: ragged tiles, enough of them for the walk of 8 at k >= 12; a few rows beyond 8
-    # slots in the CSR forms; X and Y at odd element offsets; a row range that starts inside a tile; the
-    # one-vector product of SlicedEllpack sums every row in the same order with the same rounding
+    # 65 x 67 x 61 rows: ragged tiles, a walk of 8 tiles per wave in FP64 at k >= 33 and of 2 else, a few rows beyond
+    # 8 slots (which keep the other kernel) in the CSR forms; X and Y at odd element offsets, so that 16-byte lanes
+    # never divide a row; a row range that starts inside a tile; CSRScalar's one-vector product sums every row
+    # in the same order with the same rounding
     rng = np.random.default_rng(k)
     for box, longs in (((65, 67, 61), fmt == "CSRScalar"), ((9, 5, 3), True)):
         rp, c, v = W._stencil(box[::-1], [(d, 1.0) for d in ((-1, 0, 0), (0, -1, 0), (0, 0, -1), (0, 0, 0), (0, 0, 1),
@@ -178,3 +179,74 @@ def test_short_rows_equal_the_columns_one_by_one(tnl, dev, fmt, dt, k):
             eps = 2.0 ** (-50 if dt == "f64" else -21)
             assert (Y[lo:hi].double() - ref[lo:hi]).abs().max() <= eps * 8
             assert torch.equal(Y[:lo], Y0[:lo]) and torch.equal(Y[hi:], Y0[hi:])
+
+
+def test_a_long_row_among_short_ones_costs_odd_widths_no_more(tnl, dev):
+    """The walk for short rows (odd k) is not taken where a row holds more than 8 slots: k = 7 costs what k = 8 does in
+    the other kernel (which takes it at this size), give or take; in the walk the long row alone cost 3.6 times that."""
+    n, m = 300000, 20000
+    i = np.arange(n)
+    e = np.sort(np.random.default_rng(1).choice(np.arange(2, n), m, replace=False))
+    cols = [np.concatenate([[0, 1], e]), *np.stack([i[:-2], i[1:-1], i[2:]], 1), np.array([n - 2, n - 1])]
+    rp = np.zeros(n + 1, np.int32)
+    np.cumsum([len(c) for c in cols], out=rp[1:])
+    c = np.concatenate(cols).astype(np.int32)
+    v = np.random.default_rng(2).uniform(-1, 1, len(c))
+    A = tnl.SparseMatrix.from_csr(rp, c, v, format="CSRScalar", dtype="f64")
+    took = {}
+    for k in (7, 8):
+        X = torch.tensor(np.random.default_rng(k).uniform(-1, 1, (n, k)), device=dev)
+        Y = torch.zeros_like(X)
+        for r in range(4):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            A.vectorProductMulti(X, Y)
+            e1.record()
+            e1.synchronize()
+            took[k] = min(took.get(k, 1e9), e0.elapsed_time(e1))
+        want = torch.zeros(n, dtype=torch.float64, device=dev)
+        A.vectorProduct(X[:, k - 1].contiguous(), want)
+        assert torch.equal(Y[:, k - 1], want)
+    assert took[7] < 2 * took[8], took
+
+
+@pytest.mark.parametrize("fmt,dt,k,box,aligned,longs", [
+    ("SlicedEllpack", "f64", 16, (101, 100, 83), True, 0),   # 16-byte lanes, 8 tiles per wave from 100000 tiles on
+    ("SlicedEllpack", "f64", 16, (100, 99, 79), True, 0),    # the same below that: the other kernel
+    ("SlicedEllpack", "f64", 3, (1001, 1003, 1), False, 0),  # two lanes a row, four slots a loader
+    ("Ellpack", "f64", 3, (1001, 1003, 1), False, 0),
+    ("SlicedEllpack", "f32", 33, (65, 67, 93), False, 0),    # 8 tiles per wave in FP32
+    ("CSRScalar", "f64", 7, (65, 67, 61), False, 0),
+    ("CSRScalar", "f32", 5, (65, 67, 61), True, 0),
+    ("SlicedEllpack", "f64", 7, (65, 67, 61), False, 3),     # rows beyond 8 slots: the other kernel
+    ("Ellpack", "f32", 9, (65, 67, 61), False, 3),
+])
+def test_each_rule_of_the_short_row_walk(tnl, dev, fmt, dt, k, box, aligned, longs):
+    """Every column equals the one-vector product of the same rows bit for bit, whole and over a ragged range."""
+    d = [(-1, 0, 0), (0, -1, 0), (0, 0, -1), (0, 0, 0), (0, 0, 1), (0, 1, 0), (1, 0, 0)]
+    rp, c, v = W._stencil(box, [(q, 1.0) for q in d if box[2] > 1 or q[2] == 0])
+    n = len(rp) - 1
+    rng = np.random.default_rng(k)
+    if longs:
+        at = rng.choice(n, longs, replace=False)
+        key = np.repeat(np.arange(n, dtype=np.int64), np.diff(rp)) * n + c
+        key = np.unique(np.concatenate([key] + [r * n + rng.choice(n, 13) for r in at.astype(np.int64)]))
+        c = (key % n).astype(np.int32)
+        np.cumsum(np.bincount(key // n, minlength=n), out=rp[1:])
+    v = rng.uniform(-1, 1, len(c))
+    td = torch.float64 if dt == "f64" else torch.float32
+    A = tnl.SparseMatrix.from_csr(rp, c, v, format=fmt, dtype=dt)
+    B = tnl.SparseMatrix.from_csr(rp, c, v, format="CSRScalar", dtype=dt)
+    off = 0 if aligned else 1
+    X = torch.rand(n * k + off, dtype=td, device=dev, generator=torch.Generator(dev).manual_seed(k))[off:].view(n, k)
+    Y = torch.full((n * k + off,), float("nan"), dtype=td, device=dev)[off:].view(n, k)
+    A.vectorProductMulti(X, Y)
+    lo, hi = 5, n - 6
+    Z = torch.full((n * k + off,), 2.0, dtype=td, device=dev)[off:].view(n, k)
+    A.vectorProductMulti(X, Z, 1.0, 0.0, lo, hi)
+    y = torch.zeros(n, dtype=td, device=dev)
+    for j in range(k):
+        B.vectorProduct(X[:, j].contiguous(), y)
+        assert torch.equal(Y[:, j], y), j
+        assert torch.equal(Z[lo:hi, j], y[lo:hi]), j
+    assert (Z[:lo] == 2).all() and (Z[hi:] == 2).all()

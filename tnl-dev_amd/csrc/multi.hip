@@ -213,8 +213,7 @@ struct Packed
    typedef Y type __attribute__( ( ext_vector_type( VW ), aligned( sizeof( Y ) ) ) );
 };
 
-// The product for rows of up to kMultiChunk slots (longer ones take the rest of their slots in a loop
-// of their own).  Bound by latency before it is bound by bytes: in multiProductKernel a wave lives
+// The product where no row has more than kMultiChunk slots.  Bound by latency before it is bound by bytes: in multiProductKernel a wave lives
 // for one row per L lanes, through three dependent trips to memory (row, slots, X).  Here a
 // wave walks `tiles` tiles of 64 / L rows with the next tile's slots and the one after's row
 // loaded ahead, and X of the next tile under way while it sums this one.  A tile's slots are
@@ -237,7 +236,6 @@ __global__ __launch_bounds__( 256 ) void multiShortKernel( View view, const int3
    using VY = typename Packed< Y, VW >::type;
    __shared__ __align__( 16 ) int32_t sc[ kWaves ][ 2 ][ RW * S ];
    __shared__ __align__( 16 ) A sv[ kWaves ][ 2 ][ RW * S ];
-   __shared__ int32_t sn[ kWaves ][ 2 ][ RW ];
    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
    const int loadRow = lane % RW, loadSlot = lane / RW;  // as a loader: slots loadSlot, loadSlot + L, ...
    const int myRow = lane / L, jq = lane % L;            // as a summer
@@ -262,18 +260,17 @@ __global__ __launch_bounds__( 256 ) void multiShortKernel( View view, const int3
    {
       int32_t c[ PL ];
       V v[ PL ];
-      int32_t size;
    };
    auto loadSlots = [ & ]( RowRun m, int64_t base ) {
       Slots s;
-      s.size = base + loadRow < last ? runSize( view, m ) : 0;
+      const int32_t size = base + loadRow < last ? runSize( view, m ) : 0;
       const int64_t start = runStart( view, m, base + loadRow );
 #pragma unroll
       for( int j = 0; j < PL; j++ ) {
          const int l = loadSlot + j * L;
          s.c[ j ] = -1;
          s.v[ j ] = V( 0.0f );
-         if( l < S && l < s.size ) {
+         if( l < S && l < size ) {
             const int64_t g = start + step * l;
             s.c[ j ] = __builtin_nontemporal_load( col + g );
             s.v[ j ] = val[ g ];
@@ -291,8 +288,6 @@ __global__ __launch_bounds__( 256 ) void multiShortKernel( View view, const int3
             sv[ wave ][ buf ][ loadRow * S + l ] = toCompute( s.v[ j ], A() );
          }
       }
-      if( loadSlot == 0 )
-         sn[ wave ][ buf ][ loadRow ] = s.size;
       waveSync();
    };
    struct Gathered
@@ -322,20 +317,6 @@ __global__ __launch_bounds__( 256 ) void multiShortKernel( View view, const int3
 #pragma unroll
          for( int i = 0; i < VW; i++ )
             sum[ i ] = c >= 0 ? mulAddExact( sum[ i ], a, (A) g.x[ u ][ i ] ) : sum[ i ];
-      }
-      const int32_t len = sn[ wave ][ buf ][ myRow ];
-      if( len > S ) {
-         for( int32_t l = S; l < len; l++ ) {
-            const int64_t e = view.global( (int32_t) r, l );
-            const int32_t c = col[ e ];
-            if( c >= 0 ) {
-               const A a = toCompute( val[ e ], A() );
-               const VY xv = *reinterpret_cast< const VY* >( xs + (int64_t) c * k );
-#pragma unroll
-               for( int i = 0; i < VW; i++ )
-                  sum[ i ] = mulAddExact( sum[ i ], a, (A) xv[ i ] );
-            }
-         }
       }
       if( ! mine || r >= last )
          return;
@@ -420,7 +401,9 @@ void launchMultiShort( const Matrix& M, const View& view, int32_t k, const Y* X,
 // 16 110 / 110; CSRScalar FP64 k = 3 on 127 x 150 x 93 67 / 69, FP32 k = 3 on 128^3 43 / 61.  So it
 // takes the widths that 16-byte lanes do not divide (k = 3 only where FP64 slots lie slice by slice, from a
 // million rows on), and from four lanes a row (two FP64 columns each) on where there are rows enough to
-// walk.
+// walk.  Rows beyond kMultiChunk slots would hold up a wave's whole walk: finished in a loop of their own here, one
+// row of 20000 slots among 300000 of 3 cost 6343 us instead of 1736 (k = 7), lognormal rows of 6 on average 702
+// instead of 271.
 template< int KP, typename V, typename A, typename Y >
 bool launchShort( const Matrix& M, int32_t k, const Y* X, Y* Yv, double alpha, double beta, int32_t first, int32_t last,
                   bool wide, hipStream_t st )
@@ -435,7 +418,7 @@ bool launchShort( const Matrix& M, int32_t k, const Y* X, Y* Yv, double alpha, d
    if( KP == 4 && ( sizeof( Y ) != 8 || kindOf( M.format ) == KIND_CSR || rows < 1000000 ) )
       return false;
    if constexpr( L >= 2 ) {
-      if( M.cols == 0 || M.meta.allocated > (int64_t) kMultiChunk * M.rows )
+      if( M.cols == 0 || M.rowMost > kMultiChunk )
          return false;
       bool taken = false;
       withView( M, [ & ]( auto view ) {
