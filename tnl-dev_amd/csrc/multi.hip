@@ -35,7 +35,7 @@ int64_t multiChunk( const Matrix& M, int64_t blocks, int64_t rowsPerBlock, int64
    const int64_t whole = std::max< int64_t >( 1, ( blocks + kXcds - 1 ) / kXcds );
    // (ChunkedEllpack's and BiEllpack's kernels are bound by their index maps: 328 us contiguous against 342)
    const int kind = kindOf( M.format );
-   if( kind == KIND_CHUNKED || kind == KIND_BIELLPACK || M.reach <= 0 || 3 * M.reach * rowBytes <= ( 1 << 20 ) )
+   if( kind == KIND_CHUNKED || kind == KIND_BIELLPACK || M.reach <= 0 || 3 * (int64_t) M.reach * rowBytes <= ( 1 << 20 ) )
       return whole;
    return std::min( whole, std::max< int64_t >( 1, ( M.reach / kXcds + rowsPerBlock - 1 ) / rowsPerBlock ) );
 }
