@@ -459,6 +459,13 @@ void buildSchedule( Ilu0::Sweep& s, const std::vector< int32_t >& level, const s
       int32_t e = l + 1;
       while( ! wide && e < nl && s.levels[ e + 1 ] - s.levels[ e ] <= kNarrowLevel )
          e++;
+      // a workgroup for the largest level of the run, two rows per lane: every wave of it issues the loads of every
+      // step, rows or not, and a CU issues them one after another
+      int32_t rows = 0;
+      for( int32_t lv = l; lv < e; lv++ )
+         rows = std::max( rows, s.levels[ lv + 1 ] - s.levels[ lv ] );
+      const int32_t block = std::min( kRunBlock, ( rows + kSliceRows - 1 ) / kSliceRows * kWave );
+      const int32_t stepRows = 2 * block;
       const int32_t runFirst = s.levels[ l ], firstStep = (int32_t) steps.size() / 4, firstSlice = (int32_t) slices.size() / 4;
       for( int32_t lv = l; lv < e; lv++ ) {
          const int32_t begin = s.levels[ lv ], end = s.levels[ lv + 1 ];
@@ -466,8 +473,8 @@ void buildSchedule( Ilu0::Sweep& s, const std::vector< int32_t >& level, const s
          // level, and no more than kRing positions before this level's end.  (A second entry of U
          // at the row's own column takes the value from before the row is solved: not in the ring.)
          const int32_t ringFrom = wide ? s.positions : std::max( runFirst, end - kRing );
-         for( int32_t p = begin; p < end; p += kStepRows ) {
-            const int32_t last = std::min( end, p + kStepRows );
+         for( int32_t p = begin; p < end; p += stepRows ) {
+            const int32_t last = std::min( end, p + stepRows );
             int32_t flags = last == end ? kLastOfLevel : 0;
             for( int32_t k = p; k < last; k++ ) {
                const int32_t* c = len[ k ] > 0 ? columns( order[ k ] ) : nullptr;
@@ -493,7 +500,7 @@ void buildSchedule( Ilu0::Sweep& s, const std::vector< int32_t >& level, const s
       while( ! wide && ( (int32_t) ( steps.size() / 4 ) - firstStep ) % D )
          steps.insert( steps.end(), { runFirst, 0, firstSlice, 0 } );
       s.launches.push_back( { l, e, firstStep, (int32_t) ( steps.size() / 4 ) - firstStep, firstSlice,
-                              (int32_t) ( slices.size() / 4 ) - firstSlice, wide } );
+                              (int32_t) ( slices.size() / 4 ) - firstSlice, block, wide } );
       l = e;
    }
    s.nslices = (int32_t) slices.size() / 4;
@@ -555,7 +562,7 @@ void runSweep( const Ilu0::Sweep& s, T* x, Gate gate, hipStream_t st )
          sweepLevelKernel< UPPER, T ><<< gridFor( 2 * L.slices, kIluBlock / kWave ), kIluBlock, 0, st >>>(
             f, L.firstSlice, L.slices, s.levels[ L.firstLevel ], s.levels[ L.lastLevel ], x, gate );
       else
-         sweepRunKernel< UPPER, W, D, T ><<< 1, kRunBlock, 0, st >>>( f, L.firstStep, L.steps, x, gate );
+         sweepRunKernel< UPPER, W, D, T ><<< 1, L.block, 0, st >>>( f, L.firstStep, L.steps, x, gate );
    }
    TNLHIP_CHECK( hipGetLastError() );
 }

@@ -15,6 +15,7 @@ struct Ilu0
       int32_t firstLevel, lastLevel;  // [first, last)
       int32_t firstStep, steps;
       int32_t firstSlice, slices;
+      int32_t block;  // lanes of a run's workgroup
       bool wide;
    };
    // a triangular factor in level order
