@@ -401,8 +401,9 @@ def _ilu_matrix(kind):
         n = 45000
         per = [np.unique(np.concatenate([[i - 1500], rng.integers(0, i - 1500, 2)])) if i > 1500 else np.array([], int)
                for i in range(n)]
-    else:  # "wide levels": levels on both sides of 4096 rows
-        sizes = [4096, 4097, 3, 1, 1025, 6000, 4095, 64]
+    else:  # levels on both sides of 4096 rows, or of the 1024 from which far columns make a launch of a level
+        sizes = ([4096, 4097, 3, 1, 1025, 6000, 4095, 64] if kind == "wide levels" else
+                 [4000] * 4 + [3000, 1024, 1025, 2, 130, 1026, 1500, 1000, 2000])
         start = np.concatenate([[0], np.cumsum(sizes)])
         n, per = int(start[-1]), []
         for lv, size in enumerate(sizes):
@@ -423,7 +424,7 @@ def _ilu_matrix(kind):
     return rp, np.concatenate(cols), np.concatenate(vals)
 
 
-@pytest.mark.parametrize("kind", ["chain", "long rows", "far columns", "wide levels"])
+@pytest.mark.parametrize("kind", ["chain", "long rows", "far columns", "wide levels", "far levels"])
 def test_ilu0_sweep_paths_follow_the_oracle(tnl, dev, kind):
     """The triangular sweeps give TNL's bits on every path (rows longer than the fetched entries, a
     second entry on the diagonal, columns older than the LDS ring, one-row and device-wide levels),
@@ -438,6 +439,55 @@ def test_ilu0_sweep_paths_follow_the_oracle(tnl, dev, kind):
     np.testing.assert_allclose(hist[:3], ref["history"][:3], rtol=1e-9)
     _, _, _, h32, _ = _run_device_solver(tnl, dev, "bicgstab", rp, c, v, b, fmt="CSRScalar", dtype="f32", **kw)
     np.testing.assert_allclose(h32[:2], ref["history"][:2], rtol=2e-3)  # FP32 factors and vectors
+
+
+def _levelled(levels, per, entries):
+    """`levels` levels of `per` rows in both sweeps, each row with `entries` columns anywhere in the levels before."""
+    rng = np.random.default_rng(2)
+    n = levels * per
+    i = np.arange(per, n)
+    low = (rng.random((len(i), entries)) * (i // per * per)[:, None]).astype(np.int64)
+    low[:, 0] = i - per
+    r = np.concatenate([np.arange(n), np.repeat(i, entries), i - per])
+    c = np.concatenate([np.arange(n), low.ravel(), i])
+    key, first = np.unique(r * n + c, return_index=True)
+    v = np.concatenate([np.full(n, 2.0 * entries), rng.uniform(-1, 1, low.size + len(i))])[first]
+    rp = np.zeros(n + 1, np.int32)
+    np.cumsum(np.bincount(key // n, minlength=n), out=rp[1:])
+    return rp, (key % n).astype(np.int32), v
+
+
+def _ilu_ms_per_level(tnl, dev, m, levels):
+    rp, c, v = m
+    b = t(W.uniform_vector(len(rp) - 1, 3), dev)
+    s = tnl.getLinearSolver("bicgstab")
+    s.setMatrix(tnl.SparseMatrix.from_csr(rp, c, v, format="CSRAdaptive", dtype="f64"))
+    s.setup(convergence_residue=1e-300, max_iterations=4, preconditioner=2)
+    best = 1e9
+    for _ in range(3):  # the first one builds the factors
+        x = torch.zeros_like(b)
+        torch.cuda.synchronize()
+        start = time.perf_counter()
+        s.solve(b, x)
+        best = min(best, 1e3 * (time.perf_counter() - start))
+    return best / levels
+
+
+def test_ilu0_sweep_cost_follows_the_levels(tnl, dev):
+    """What a level of a triangular sweep costs: a level of one row a fraction of one of 1400 (a run's workgroup is as
+    large as its levels; 0.3 measured, 0.8 with 16 waves for every run), and 2500 rows whose columns lie anywhere before
+    them no more than 6000 such rows, which are a launch (0.9 measured, 2.6 in a run)."""
+    n = 4000
+    i = np.arange(n)
+    r, c = np.concatenate([i[1:], i, i[:-1]]), np.concatenate([i[1:] - 1, i, i[:-1] + 1])
+    o = np.lexsort((c, r))
+    rp = np.zeros(n + 1, np.int32)
+    np.cumsum(np.bincount(r, minlength=n), out=rp[1:])
+    chain = _ilu_ms_per_level(tnl, dev, (rp, c[o].astype(np.int32), np.where(c == r, 4.0, -1.0)[o]), n)
+    grid = _ilu_ms_per_level(tnl, dev, W.laplacian_3d(64), 190)
+    assert chain < 0.5 * grid, (chain, grid)
+    few, many = (_ilu_ms_per_level(tnl, dev, _levelled(40, rows, 13), 40) for rows in (2500, 6000))
+    assert few < 1.6 * many, (few, many)
 
 
 def test_ilu0_refuses_rows_without_an_upper_entry(tnl, dev):

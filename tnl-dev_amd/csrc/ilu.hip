@@ -41,6 +41,7 @@ constexpr int kRunBlock = 1024;         // one workgroup of 16 waves for runs of
 constexpr int32_t kStepRows = 2 * kRunBlock;
 constexpr int32_t kSliceRows = 2 * kWave;
 constexpr int32_t kNarrowLevel = 4096;  // levels of at most this many rows are taken in runs
+constexpr int32_t kFarLevel = 1024;     // and these where some entry is older than the ring
 constexpr int32_t kNarrowFactor = 1024; // likewise in the factorization
 constexpr int32_t kRing = 16384;        // solution entries kept in LDS by a run (128 KiB in FP64)
 static_assert( kRing >= 2 * kNarrowLevel && ( kRing & ( kRing - 1 ) ) == 0 && kRing < 65536,
@@ -223,20 +224,33 @@ __global__ __launch_bounds__( kIluBlock ) void permuteKernel( int32_t n, const i
       dst[ k ] = src[ index[ k ] ];
 }
 
-// The entries of a row from entry `from` on in the rest arrays: sub( column, value ) for each, left
-// to right; `start` is the start of the row's half of its slice.
-template< typename T, typename F >
-__device__ __forceinline__ void restOfRow( const SweepView< T >& f, int32_t start, int32_t from, int32_t n, F&& sub )
+// Subtracts the entries of a row from entry `from` on, which are in the rest arrays, from acc, left to
+// right; `start` is the start of the row's half of its slice, solved( column ) a solution entry.  The
+// loads of U entries go out together: one by one each took two trips to memory (27-point 60^3, BiCGStab:
+// 14.3 -> 8.2 ms an iteration).
+template< int U, typename T, typename F >
+__device__ __forceinline__ void restOfRow( const SweepView< T >& f, int32_t start, int32_t from, int32_t n, T& acc,
+                                           F&& solved )
 {
    const int lane = threadIdx.x % kWave;
    int32_t e = start;
-   for( int32_t l = from;; l++ ) {
-      const unsigned long long on = __ballot( l < n );
-      if( ! on )
-         break;
-      if( l < n )
-         sub( f.restCol[ e + lane ], f.restVal[ e + lane ] );
-      e += __popcll( on );
+   for( int32_t l = from; __any( l < n ); l += U ) {
+      int32_t c[ U ];
+      T v[ U ], xv[ U ];
+#pragma unroll
+      for( int u = 0; u < U; u++ ) {
+         // a lane without the entry reads the first one of the half slice
+         const int32_t at = l + u < n ? e + lane : start;
+         c[ u ] = f.restCol[ at ];
+         v[ u ] = f.restVal[ at ];
+         e += __popcll( __ballot( l + u < n ) );
+      }
+#pragma unroll
+      for( int u = 0; u < U; u++ )
+         xv[ u ] = solved( c[ u ] );
+#pragma unroll
+      for( int u = 0; u < U; u++ )
+         acc = l + u < n ? mulSubExact( acc, v[ u ], xv[ u ] ) : acc;
    }
 }
 
@@ -253,8 +267,8 @@ __global__ __launch_bounds__( kIluBlock ) void sweepLevelKernel( SweepView< T > 
       const int32_t p = begin + h / 2 * kSliceRows + 2 * lane + h % 2;
       const bool mine = p < end;
       T acc = mine ? x[ p ] : (T) 0;
-      restOfRow( f, f.sliceRest[ 2 * firstSlice + h ], 0, mine ? f.len[ p ] : 0,
-                 [ & ]( int32_t c, T v ) { acc = mulSubExact( acc, v, x[ ~c ] ); } );
+      restOfRow< 8 >( f, f.sliceRest[ 2 * firstSlice + h ], 0, mine ? f.len[ p ] : 0, acc,
+                      [ & ]( int32_t c ) { return x[ ~c ]; } );
       if( mine )
          x[ p ] = UPPER ? acc / f.diag[ p ] : acc;
    }
@@ -351,15 +365,9 @@ __global__ __launch_bounds__( kRunBlock ) void sweepRunKernel( SweepView< T > f,
          if( wave * kWave < q.pairs ) {
             for( int odd = 0; odd < 2; odd++ ) {
                T a = odd ? acc[ 1 ] : acc[ 0 ];
-               restOfRow( f, f.sliceRest[ 2 * ( q.slice + wave ) + odd ], q.flags & kAllInRest ? 0 : W,
-                          mine ? f.len[ q.first + 2 * tid + odd ] : 0, [ & ]( int32_t c, T v ) {
-                             T xv;
-                             if( c >= 0 )
-                                xv = ring[ c ];
-                             else
-                                xv = x[ ~c ];
-                             a = mulSubExact( a, v, xv );
-                          } );
+               restOfRow< W <= 4 ? 4 : 8 >( f, f.sliceRest[ 2 * ( q.slice + wave ) + odd ], q.flags & kAllInRest ? 0 : W,
+                          mine ? f.len[ q.first + 2 * tid + odd ] : 0, a,
+                          [ & ]( int32_t c ) { return c >= 0 ? ring[ c ] : x[ ~c ]; } );
                if( odd )
                   acc[ 1 ] = a;
                else
@@ -454,40 +462,35 @@ void buildSchedule( Ilu0::Sweep& s, const std::vector< int32_t >& level, const s
    }
    s.rest = 0;
    s.launches.clear();
-   for( int32_t l = 0; l < nl; ) {
-      const bool wide = s.levels[ l + 1 ] - s.levels[ l ] > kNarrowLevel;
-      int32_t e = l + 1;
-      while( ! wide && e < nl && s.levels[ e + 1 ] - s.levels[ e ] <= kNarrowLevel )
-         e++;
-      // a workgroup for the largest level of the run, two rows per lane: every wave of it issues the loads of every
-      // step, rows or not, and a CU issues them one after another
-      int32_t rows = 0;
-      for( int32_t lv = l; lv < e; lv++ )
-         rows = std::max( rows, s.levels[ lv + 1 ] - s.levels[ lv ] );
-      const int32_t block = std::min( kRunBlock, ( rows + kSliceRows - 1 ) / kSliceRows * kWave );
-      const int32_t stepRows = 2 * block;
+   auto rowsOf = [ & ]( int32_t l ) { return s.levels[ l + 1 ] - s.levels[ l ]; };
+   // The positions a step of level l finds in the ring of a run that starts at position runFirst: solved by the
+   // run in an earlier level, and no more than kRing positions before this level's end.  (A second entry of U
+   // at the row's own column takes the value from before the row is solved: not in the ring.)
+   auto ringFrom = [ & ]( int32_t l, int32_t runFirst ) { return std::max( runFirst, s.levels[ l + 1 ] - kRing ); };
+   // whether some of the first W entries of rows [ p, last ) of level l are not in that ring
+   auto outside = [ & ]( int32_t l, int32_t p, int32_t last, int32_t runFirst ) {
+      const int32_t begin = s.levels[ l ], oldest = ringFrom( l, runFirst );
+      for( int32_t k = p; k < last; k++ ) {
+         const int32_t* c = len[ k ] > 0 ? columns( order[ k ] ) : nullptr;
+         for( int32_t j = 0; j < std::min( len[ k ], W ); j++ )
+            if( position[ c[ j ] ] < oldest || position[ c[ j ] ] >= begin )
+               return true;
+      }
+      return false;
+   };
+   // the steps and slices of levels [ l, e ); flags: of each step, nullptr where every entry is in the rest arrays
+   auto addLaunch = [ & ]( int32_t l, int32_t e, int32_t block, const int32_t* flags ) {
       const int32_t runFirst = s.levels[ l ], firstStep = (int32_t) steps.size() / 4, firstSlice = (int32_t) slices.size() / 4;
       for( int32_t lv = l; lv < e; lv++ ) {
          const int32_t begin = s.levels[ lv ], end = s.levels[ lv + 1 ];
-         // the positions a step of this level finds in the ring: solved by the run in an earlier
-         // level, and no more than kRing positions before this level's end.  (A second entry of U
-         // at the row's own column takes the value from before the row is solved: not in the ring.)
-         const int32_t ringFrom = wide ? s.positions : std::max( runFirst, end - kRing );
-         for( int32_t p = begin; p < end; p += stepRows ) {
-            const int32_t last = std::min( end, p + stepRows );
-            int32_t flags = last == end ? kLastOfLevel : 0;
-            for( int32_t k = p; k < last; k++ ) {
-               const int32_t* c = len[ k ] > 0 ? columns( order[ k ] ) : nullptr;
-               for( int32_t j = 0; j < std::min( len[ k ], W ) && ! ( flags & kAllInRest ); j++ )
-                  if( position[ c[ j ] ] < ringFrom || position[ c[ j ] ] >= begin )
-                     flags |= kAllInRest;
-               if( len[ k ] > W )
-                  flags |= kLongRow;
-            }
-            const int32_t from = flags & kAllInRest ? 0 : W, step = (int32_t) steps.size() / 4;
-            steps.insert( steps.end(), { p, ( last - p ) / 2, (int32_t) slices.size() / 4, flags } );
+         const int32_t oldest = flags ? ringFrom( lv, runFirst ) : s.positions;
+         for( int32_t p = begin; p < end; p += 2 * block ) {
+            const int32_t last = std::min( end, p + 2 * block );
+            const int32_t flag = flags ? *flags++ : kAllInRest;
+            const int32_t from = flag & kAllInRest ? 0 : W, step = (int32_t) steps.size() / 4;
+            steps.insert( steps.end(), { p, ( last - p ) / 2, (int32_t) slices.size() / 4, flag } );
             for( int32_t q = p; q < last; q += kSliceRows ) {
-               slices.insert( slices.end(), { q, step, ringFrom, begin } );
+               slices.insert( slices.end(), { q, step, oldest, begin } );
                for( int odd = 0; odd < 2; odd++ ) {
                   sliceRest.push_back( s.rest );
                   for( int32_t k = q + odd; k < std::min( q + kSliceRows, last ); k += 2 )
@@ -497,11 +500,44 @@ void buildSchedule( Ilu0::Sweep& s, const std::vector< int32_t >& level, const s
          }
       }
       // a run takes its steps in rounds of D: steps without rows fill the last one
-      while( ! wide && ( (int32_t) ( steps.size() / 4 ) - firstStep ) % D )
+      while( flags && ( (int32_t) ( steps.size() / 4 ) - firstStep ) % D )
          steps.insert( steps.end(), { runFirst, 0, firstSlice, 0 } );
       s.launches.push_back( { l, e, firstStep, (int32_t) ( steps.size() / 4 ) - firstStep, firstSlice,
-                              (int32_t) ( slices.size() / 4 ) - firstSlice, block, wide } );
-      l = e;
+                              (int32_t) ( slices.size() / 4 ) - firstSlice, block, ! flags } );
+   };
+   // A level that is a launch of its own: more rows than a run takes, or more than kFarLevel of them with an
+   // entry older than the ring, which a run's one CU would fetch from memory.  us per iteration of BiCGStab (four
+   // sweeps), 40 levels that draw on all before them, in the run / as launches: 4000 rows of 3 entries 1759 / 1103, 2500 of
+   // 13 3607 / 1406, 1100 of 13 1312 / 1095; at 900 rows of 13, in the run 1050.
+   auto wide = [ & ]( int32_t l ) {
+      return rowsOf( l ) > kNarrowLevel ||
+             ( rowsOf( l ) > kFarLevel && outside( l, s.levels[ l ], s.levels[ l + 1 ], 0 ) );
+   };
+   for( int32_t l = 0; l < nl; ) {
+      int32_t e = l, rows = 0;
+      for( ; e < nl && ! wide( e ); e++ )
+         rows = std::max( rows, rowsOf( e ) );
+      if( e > l ) {
+         // a workgroup for the largest level of the run, two rows per lane: every wave of it issues the loads of
+         // every step, rows or not, and a CU issues them one after another (tridiagonal matrix of 20000 rows,
+         // BiCGStab: 129 ms an iteration with 16 waves, 48 ms)
+         const int32_t block = std::min( kRunBlock, ( rows + kSliceRows - 1 ) / kSliceRows * kWave );
+         std::vector< int32_t > flags;
+         for( int32_t lv = l; lv < e; lv++ ) {
+            // wide() has seen that the ring holds what its rows need, if it began that early
+            const bool inside = rowsOf( lv ) > kFarLevel && ringFrom( lv, s.levels[ l ] ) == ringFrom( lv, 0 );
+            for( int32_t p = s.levels[ lv ]; p < s.levels[ lv + 1 ]; p += 2 * block ) {
+               const int32_t last = std::min( s.levels[ lv + 1 ], p + 2 * block );
+               flags.push_back( ( last == s.levels[ lv + 1 ] ? kLastOfLevel : 0 ) |
+                                ( ! inside && outside( lv, p, last, s.levels[ l ] ) ? kAllInRest : 0 ) |
+                                ( len[ p ] > W ? kLongRow : 0 ) );  // the longest row is the first one
+            }
+         }
+         addLaunch( l, e, block, flags.data() );
+      }
+      if( e < nl )
+         addLaunch( e, e + 1, kRunBlock, nullptr );
+      l = e + 1;
    }
    s.nslices = (int32_t) slices.size() / 4;
    s.order.upload( order, st );
