@@ -365,6 +365,40 @@ def test_iteration_limits_of_fused_solves(tnl, dev, method, most):
     np.testing.assert_allclose(x, ref["x"], rtol=0, atol=1e-7 * np.abs(ref["x"]).max() + 1e-300)
 
 
+def _solve_us(tnl, dev, method, dtype, most, repeats):
+    """Shortest time of a solve cut off after `most` iterations, and the iterations it made."""
+    rp, c, v = W.laplacian_2d(205)
+    A = tnl.SparseMatrix.from_csr(rp, c, v, format="SlicedEllpack", dtype=dtype)
+    s = tnl.getLinearSolver(method)
+    s.setMatrix(A)
+    s.setup(convergence_residue=1e-300, max_iterations=most)
+    b = t(W.uniform_vector(len(rp) - 1, 3), dev, A.vector_dtype)
+    best = 1e9
+    for _ in range(repeats):
+        x = torch.zeros_like(b)
+        torch.cuda.synchronize()
+        start = time.perf_counter()
+        s.solve(b, x)
+        best = min(best, 1e6 * (time.perf_counter() - start))
+    return best, s.getIterations()
+
+
+@pytest.mark.parametrize("method", ["cg", "bicgstab"])
+def test_a_solve_of_the_eager_batches_builds_no_graph(tnl, dev, method):
+    """The launches that close the last of 4 and 8 iterations belong to the eager batches: cut off after 11 (one more is
+    counted) a solve costs about 1.05 times the 10, with a graph built for the closing launches 1.6 times."""
+    ten, eleven = (_solve_us(tnl, dev, method, "f64", most, 20)[0] for most in (10, 11))
+    assert eleven < 1.3 * ten, (ten, eleven)
+
+
+def test_restarts_do_not_queue_ahead_of_each_other(tnl, dev):
+    """FP32 BiCGStab that cannot get any lower restarts again and again; an iteration then costs about 1.3 times one
+    of the FP64 solve, which does not (1.75 times with 64 iterations queued behind every restart)."""
+    (low, its), (high, n) = (_solve_us(tnl, dev, "bicgstab", d, 1000, 4) for d in ("f32", "f64"))
+    assert its >= 1000 and n >= 1000
+    assert low / its < 1.5 * high / n, (low / its, high / n)
+
+
 @pytest.mark.parametrize("fmt", ["SlicedEllpack", "CSRAdaptive"])
 def test_ilu0_wide_levels_follow_the_oracle(tnl, dev, fmt):
     """ILU(0) on the 64^3 Laplacian: the anti-diagonal planes hold up to 3072 rows, so the

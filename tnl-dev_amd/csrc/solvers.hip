@@ -535,6 +535,8 @@ void runChunks( SolverImpl& S, Iter&& iteration )
 // The same for solves whose fused passes alternate between two sets of buffers: iteration( odd )
 // queues one iteration, `next` is the number of the next one and decides the set.  A solve that
 // stops with flags[1] set asks the host for `restart()` and goes on with the iteration that stopped.
+// An iteration closes the one before it, so a solve of k iterations queues k + 1: the eager batches and
+// the replays end one later than runChunks' (with 12 eager iterations a solve of 12 built a graph: 286 -> 489 us).
 template< typename Iter, typename Restart >
 void runAlternating( SolverImpl& S, Iter&& iteration, Restart&& restart )
 {
@@ -551,14 +553,14 @@ void runAlternating( SolverImpl& S, Iter&& iteration, Restart&& restart )
             (void) hipGraphDestroy( g );
       }
    } graph;
-   int64_t next = 0;
+   int64_t next = 0, phase = -1;  // the graph's first iteration is odd or even
    // the iteration after the last one allowed only checks the stopping rule
    const int64_t limit = (int64_t) S.params.max_iterations + 3;
    int reps = 1, chunk = 16;
    while( true ) {
-      if( next < 12 || next % 2 != 0 || ! S.params.use_graph ) {
-         int64_t end = next < 4 ? 4 : 12;
-         if( next >= 12 ) {
+      if( next < 13 || ( graph.e && next % 2 != phase ) || ! S.params.use_graph ) {
+         int64_t end = next < 5 ? 5 : 13;
+         if( next >= 13 ) {
             end = S.params.use_graph ? next + 1 : next + chunk;
             chunk = std::min( chunk * 2, 64 );
          }
@@ -567,10 +569,11 @@ void runAlternating( SolverImpl& S, Iter&& iteration, Restart&& restart )
       }
       else {
          if( ! graph.e ) {
+            phase = next % 2;
             TNLHIP_CHECK( hipStreamBeginCapture( S.stream, hipStreamCaptureModeThreadLocal ) );
             try {
                for( int k = 0; k < kGraphIters; k++ )
-                  iteration( k % 2 != 0 );
+                  iteration( ( phase + k ) % 2 != 0 );
             }
             catch( ... ) {
                hipGraph_t broken = nullptr;
@@ -590,6 +593,8 @@ void runAlternating( SolverImpl& S, Iter&& iteration, Restart&& restart )
       if( h.flags[ 0 ] && h.flags[ 1 ] ) {
          restart();
          next = h.it;
+         reps = 1;  // one restart is often followed by another: what is queued behind it is for nothing
+         chunk = 16;
          continue;
       }
       if( h.flags[ 0 ] || next >= limit )
