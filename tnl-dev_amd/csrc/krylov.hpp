@@ -6,7 +6,7 @@
 // rows' share of the dot and stores one partial, and the operand can be formed where it is
 // gathered (p[c] = z[c] + beta p_old[c]), each row's own entry being stored for the passes that
 // follow.  The scalars come from the partials of the launch before, summed by every workgroup in
-// the same order (foldPartials*), so there are no launches for them either.  A CG iteration is then two
+// the same order (Fold), so there are no launches for them either.  A CG iteration is then two
 // launches and a BiCGStab iteration three.
 #pragma once
 
@@ -104,6 +104,12 @@ __device__ __forceinline__ bool leadLane()
 // issues the loads of the gate and of the first kFoldAhead partials per lane (all there are for up to
 // 1024), begin() adds them up.  Nothing waits in prefetch(): the gate is looked at after the sum, since
 // a launch that finds it closed has no time to lose.
+// The gate's flag is the one state field that workgroup 0 may set while other workgroups of the launch still
+// read it.  A launch that sets it may therefore be carried out by some of its workgroups only, and nothing it
+// made may be used afterwards: the launches queued behind it find the gate closed, and a restart starts from x.
+// The waves of one workgroup may see it differently, so whoever has a barrier ahead asks all of them (openKeeper)
+// or reaches it either way (the kernels that call begin() between their loads; a pass with sums is in no launch that
+// sets the flag without every workgroup returning).
 constexpr int kFoldAhead = 4;
 
 template< int W >
@@ -156,7 +162,7 @@ struct Fold
 // row( r, v, acc ) takes the product's (stored) entry of row r.  Entries that are formed on the way are
 // formed by explicit fused multiply-adds, so that every gather of an entry and its stored copy have
 // the same bits.  The state fields a workgroup needs are loaded in prefetch(), and workgroup 0
-// writes only fields that no workgroup of the same launch reads.
+// writes only fields that no other workgroup of the same launch uses, but for the stop flag (Fold).
 
 // CG's scalars for the iteration that begins (FinCgBeta) from the (r, z) partials
 struct CgNext

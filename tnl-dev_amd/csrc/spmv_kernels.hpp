@@ -34,7 +34,8 @@ __device__ __forceinline__ A madd( A acc, A a, A b )
       return acc + a * b;
 }
 
-// closed(), prefetch() and begin() in one
+// closed(), prefetch() and begin() in one; the answer is the workgroup's, whose waves may see a gate that is just
+// being closed differently and have barriers ahead of them
 template< typename Keep >
 __device__ __forceinline__ bool openKeeper( Keep& keep )
 {
@@ -42,7 +43,7 @@ __device__ __forceinline__ bool openKeeper( Keep& keep )
       return ! keep.closed();
    else {
       keep.prefetch();
-      return keep.begin();
+      return __syncthreads_and( keep.begin() );
    }
 }
 
