@@ -113,22 +113,6 @@ __device__ __forceinline__ void sumPartials( ReduceSlot slot, int grid, double* 
          const double* p = slot.partials + (int64_t) k * grid;
          double a0 = 0, a1 = 0, a2 = 0, a3 = 0;
          int j = threadIdx.x;
-         if( grid > 2 * kReduceGrid ) {
-            // the partials of a fused product (up to kMaxFusedPartials): more loads in flight
-            double a[ kSumStreams ] = {};
-            for( ; j + ( kSumStreams - 1 ) * kReduceBlock < grid; j += kSumStreams * kReduceBlock ) {
-#pragma unroll
-               for( int u = 0; u < kSumStreams; u++ )
-                  a[ u ] += p[ j + u * kReduceBlock ];
-            }
-#pragma unroll
-            for( int u = 0; u < kSumStreams; u += 4 ) {
-               a0 += a[ u ];
-               a1 += a[ u + 1 ];
-               a2 += a[ u + 2 ];
-               a3 += a[ u + 3 ];
-            }
-         }
          for( ; j + 3 * kReduceBlock < grid; j += 4 * kReduceBlock ) {
             a0 += p[ j ];
             a1 += p[ j + kReduceBlock ];
