@@ -54,19 +54,11 @@ void Matrix::uploadMetadata()
    switch( meta.kind ) {
       case KIND_CSR:
          offsets.upload( meta.offsets );
-         rowMost = waveMost = 0;
-         for( int32_t r = 0; r < rows; r += kWave ) {
-            const int32_t end = std::min( r + kWave, rows );
-            waveMost = std::max( waveMost, meta.offsets[ end ] - meta.offsets[ r ] );
-            for( int32_t k = r; k < end; k++ )
-               rowMost = std::max( rowMost, meta.offsets[ k + 1 ] - meta.offsets[ k ] );
-         }
+         waveMost = 0;
+         for( int32_t r = 0; r < rows; r += kWave )
+            waveMost = std::max( waveMost, meta.offsets[ std::min( r + kWave, rows ) ] - meta.offsets[ r ] );
          break;
-      case KIND_ELLPACK: rowMost = meta.segmentSize; break;
       case KIND_SLICED:
-         rowMost = 0;
-         for( int32_t w : meta.sliceSegmentSizes )
-            rowMost = std::max( rowMost, w );
          sliceOffsets.upload( meta.sliceOffsets );
          sliceSizes.upload( meta.sliceSegmentSizes );
          break;

@@ -418,7 +418,7 @@ bool launchShort( const Matrix& M, int32_t k, const Y* X, Y* Yv, double alpha, d
    if( KP == 4 && ( sizeof( Y ) != 8 || kindOf( M.format ) == KIND_CSR || rows < 1000000 ) )
       return false;
    if constexpr( L >= 2 ) {
-      if( M.cols == 0 || M.rowMost > kMultiChunk )
+      if( M.cols == 0 || M.meta.rowMost > kMultiChunk )
          return false;
       bool taken = false;
       withView( M, [ & ]( auto view ) {

@@ -25,6 +25,7 @@ void csrOffsets( HostSegments& s, const int32_t* caps )
    for( int32_t i = 0; i < s.n; i++ ) {
       s.offsets[ i ] = (int32_t) run;
       run += caps[ i ];
+      s.rowMost = std::max( s.rowMost, caps[ i ] );
    }
    if( run > std::numeric_limits< int32_t >::max() )
       throw Error( TNLHIP_ERROR_CAPACITY, "CSR storage exceeds the int32 index range" );
@@ -37,7 +38,7 @@ void ellpack( HostSegments& s, const int32_t* caps )
    int32_t mx = 0;
    for( int32_t i = 0; i < s.n; i++ )
       mx = std::max( mx, caps[ i ] );
-   s.segmentSize = mx;
+   s.segmentSize = s.rowMost = mx;
    s.alignedSize = ceilDiv( s.n, kEllpackAlignment ) * kEllpackAlignment;
    s.storage = s.allocated = (int64_t) s.alignedSize * s.segmentSize;
 }
@@ -57,6 +58,7 @@ void sliced( HostSegments& s, const int32_t* caps )
          total += caps[ i ];
       }
       s.sliceSegmentSizes[ sl ] = mx;
+      s.rowMost = std::max( s.rowMost, mx );
       s.sliceOffsets[ sl ] = (int32_t) off;
       off += (int64_t) mx * S;
    }
