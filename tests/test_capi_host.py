@@ -2,6 +2,8 @@
 and its host-side segments metadata is TNL's, bit for bit (no GPU needed)."""
 import os
 import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -125,3 +127,26 @@ def test_noalloc_multidot_refuses_before_touching_the_gpu(tnl):
     assert lib.tnlhip_multidot_noalloc(0, 64, 4, dummy, 32, dummy, dummy, None) == 1  # ld < n
     assert lib.tnlhip_multidot_noalloc(0, 64, 4, None, 64, dummy, dummy, None) == 1
     assert lib.tnlhip_multidot_noalloc(2, 64, 4, dummy, 64, dummy, dummy, None) == 1  # BF16 vectors
+
+
+def test_matrices_need_no_torch():
+    """The package and what it knows of a matrix (reading, converting and writing go through it) work where torch
+    cannot be imported; vectors are torch's, so products do need it."""
+    code = f"""
+import sys
+class NoTorch:
+    def find_spec(self, name, path=None, target=None):
+        if name.split(".")[0] == "torch":
+            raise ImportError(name)
+sys.meta_path.insert(0, NoTorch())
+sys.path.insert(0, {ROOT!r})
+from __graft_entry__ import load_package
+tnl = load_package()
+A = tnl.SparseMatrix.__new__(tnl.SparseMatrix)
+A._h = None
+A.info = tnl.MatrixInfo(rows=3, columns=4, value_dtype=1)
+assert A.info.rows == 3 and A.info.columns == 4 and "torch" not in sys.modules
+print("no torch")
+"""
+    done = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300)
+    assert done.returncode == 0 and "no torch" in done.stdout, done.stderr

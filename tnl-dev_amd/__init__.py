@@ -290,11 +290,11 @@ class SparseMatrix:
 
     @info.setter
     def info(self, info):
-        import torch
         self._info = info
-        # what every product checks, read from the struct once
+        # what every product checks, read from the struct once (the type by the first product: matrices are
+        # built, read and written without torch too)
         self._rows, self._columns = info.rows, info.columns
-        self._vector_dtype = {0: torch.float64, 3: torch.int32}.get(info.value_dtype, torch.float32)
+        self._vector_dtype = None
 
     @classmethod
     def from_csr(cls, row_pointers, column_indexes, values, columns=None, format="CSRScalar", dtype="f64"):
@@ -413,6 +413,9 @@ class SparseMatrix:
 
     @property
     def vector_dtype(self):
+        if self._vector_dtype is None:
+            import torch
+            self._vector_dtype = {0: torch.float64, 3: torch.int32}.get(self._info.value_dtype, torch.float32)
         return self._vector_dtype
 
     def convert(self, format, dtype=None):
@@ -505,7 +508,7 @@ class SparseMatrix:
                       firstRow=0, lastRow=0, stream=None):
         """outVector = matrixMultiplicator * A inVector + outVectorMultiplicator * outVector over rows
         [firstRow, lastRow) (lastRow 0 = all), SparseMatrix.h:1078-1085.  Asynchronous on the stream."""
-        dt = self._vector_dtype
+        dt = self._vector_dtype or self.vector_dtype
         if inVector.dtype != dt or outVector.dtype != dt:
             raise TypeError(f"vectors must be {dt}")
         if inVector.numel() != self._columns or outVector.numel() != self._rows:
