@@ -391,6 +391,24 @@ def test_a_solve_of_the_eager_batches_builds_no_graph(tnl, dev, method):
     assert eleven < 1.3 * ten, (ten, eleven)
 
 
+@pytest.mark.parametrize("method,vectors", [("cg", 4), ("bicgstab", 7)])
+def test_large_solves_keep_one_set_of_vectors(tnl, dev, method, vectors):
+    """Beyond the rows whose operands the products form, a solve allocates what it did with separate passes."""
+    rp, c, v = W.laplacian_2d(2000)
+    A = tnl.SparseMatrix.from_csr(rp, c, v, format="SlicedEllpack", dtype="f64")
+    s = tnl.getLinearSolver(method)
+    s.setMatrix(A)
+    s.setup(convergence_residue=1e-300, max_iterations=2)
+    b = t(W.uniform_vector(len(rp) - 1, 3), dev)
+    x = torch.zeros_like(b)
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    s.solve(b, x)
+    used = before - torch.cuda.mem_get_info()[0]
+    size = 8 * (len(rp) - 1)
+    assert used < (vectors + 0.9) * size, used / size
+
+
 def test_restarts_do_not_queue_ahead_of_each_other(tnl, dev):
     """FP32 BiCGStab that cannot get any lower restarts again and again; an iteration then costs about 1.3 times one
     of the FP64 solve, which does not (1.75 times with 64 iterations queued behind every restart)."""

@@ -894,8 +894,9 @@ struct CgFusedInitOp : NoScalars
 template< typename T >
 void solveCGFused( SolverImpl& S, const void* b, T* x, int dotGrid )
 {
+   const bool fuse = fuseOperand( *S.A );
    T* r = (T*) S.vec( 0 );
-   T* p[ 2 ] = { (T*) S.vec( 1 ), (T*) S.vec( 4 ) };
+   T* p[ 2 ] = { (T*) S.vec( 1 ), fuse ? (T*) S.vec( 4 ) : nullptr };
    T* Ap = (T*) S.vec( 2 );
    T* z = (T*) S.vec( 3 );
    const T* diag = S.params.preconditioner == 1 ? (const T*) S.diag.ptr : nullptr;
@@ -905,7 +906,6 @@ void solveCGFused( SolverImpl& S, const void* b, T* x, int dotGrid )
    State* st = S.state.ptr;
    const ReduceSlot dot = S.ws.slot( 1 ), upd = S.ws.slot( 2 );
    const int grid = passGrid< T >( S.n );
-   const bool fuse = fuseOperand( *S.A );
    const CgNext next{ st, S.hist.ptr, S.histCap, stop, { upd, grid } };
    const CgAlpha alpha{ st, S.hist.ptr, S.histCap, { dot, dotGrid } };
    computeNormb< T >( S, b, z );
@@ -1284,11 +1284,12 @@ struct FinBiResume
 template< typename T >
 void solveBiCGStabFused( SolverImpl& S, const void* b, T* x, int dotGrid )
 {
+   const bool fuse = fuseOperand( *S.A );
    T* r = (T*) S.vec( 0 );
    T* rast = (T*) S.vec( 1 );
    T* p[ 2 ] = { (T*) S.vec( 2 ), (T*) S.vec( 6 ) };
    T* s = (T*) S.vec( 3 );
-   T* Ap[ 2 ] = { (T*) S.vec( 4 ), (T*) S.vec( 7 ) };
+   T* Ap[ 2 ] = { (T*) S.vec( 4 ), fuse ? (T*) S.vec( 7 ) : nullptr };
    T* As = (T*) S.vec( 5 );
    const T* diag = S.params.preconditioner == 1 ? (const T*) S.diag.ptr : nullptr;
    const Gate always{ nullptr, 0 }, running{ S.state.ptr->flags, 1 };
@@ -1299,7 +1300,6 @@ void solveBiCGStabFused( SolverImpl& S, const void* b, T* x, int dotGrid )
    const BiNext next{ st, S.hist.ptr, S.histCap, S.stopRule(), eps * eps, { upd, grid } };
    const BiAlpha alpha{ st, { dot, dotGrid } };
    const BiOmega omega{ st, { om, dotGrid } };
-   const bool fuse = fuseOperand( *S.A );
    computeNormb< T >( S, b, p[ 1 ] );
    residual< T >( S, b, x, r, always );
    fusedReduceKernel< 2 ><<< grid, kReduceBlock, 0, S.stream >>>(
@@ -2860,9 +2860,11 @@ void prepare( SolverImpl& S )
    // column stride aligned to 256 bytes, as GMRES::setSize does for GPUs (GMRES.hpp:765-773)
    const int64_t per = 256 / (int64_t) S.vbytes;
    S.ld = ( S.n + per - 1 ) / per * per;
-   int nvec = 5;
+   // a fused solve that forms its operands in the products keeps two sets of them
+   const bool twoSets = S.params.preconditioner <= 1 && ! S.A->symmetric && fuseOperand( *S.A );
+   int nvec = twoSets ? 5 : 4;
    if( S.method == TNLHIP_BICGSTAB )
-      nvec = 8;
+      nvec = twoSets ? 8 : 7;
    if( S.method == TNLHIP_TFQMR )
       nvec = 8;
    if( S.method == TNLHIP_BICGSTABL ) {
