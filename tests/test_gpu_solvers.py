@@ -366,8 +366,10 @@ def test_iteration_limits_of_fused_solves(tnl, dev, method, most):
 
 
 def _solve_us(tnl, dev, method, dtype, most, repeats):
-    """Shortest time of a solve cut off after `most` iterations, and the iterations it made."""
+    """Shortest time of a solve cut off after `most` iterations, and the iterations it made; diagonally dominant, so that
+    FP32 is at its rounding level within tens of iterations."""
     rp, c, v = W.laplacian_2d(205)
+    v = np.where(v > 0, 6.5, v)
     A = tnl.SparseMatrix.from_csr(rp, c, v, format="SlicedEllpack", dtype=dtype)
     s = tnl.getLinearSolver(method)
     s.setMatrix(A)
@@ -410,11 +412,11 @@ def test_large_solves_keep_one_set_of_vectors(tnl, dev, method, vectors):
 
 
 def test_restarts_do_not_queue_ahead_of_each_other(tnl, dev):
-    """FP32 BiCGStab that cannot get any lower restarts again and again; an iteration then costs about 1.3 times one
-    of the FP64 solve, which does not (1.75 times with 64 iterations queued behind every restart)."""
+    """FP32 BiCGStab that cannot get any lower restarts again and again; an iteration then costs 1.1 times one of
+    the FP64 solve, which does not (1.36 times with up to 64 iterations queued behind every restart)."""
     (low, its), (high, n) = (_solve_us(tnl, dev, "bicgstab", d, 1000, 4) for d in ("f32", "f64"))
     assert its >= 1000 and n >= 1000
-    assert low / its < 1.5 * high / n, (low / its, high / n)
+    assert low / its < 1.24 * high / n, (low / its, high / n)
 
 
 @pytest.mark.parametrize("fmt", ["SlicedEllpack", "CSRAdaptive"])
