@@ -90,3 +90,13 @@ def test_slice_sizes_follow_the_oracle(tnl, dev, S):
     if S != 32:
         with pytest.raises(tnl.TnlHipError):
             A.save("/tmp/sliced_nondefault.tnl")
+
+
+@pytest.mark.parametrize("fmt,dtype,shape", [("Ellpack", "f64", (32, 1)), ("Ellpack", "bf16", (32, 1)),
+                                             ("SlicedEllpack", "f64", (32, 1)), ("SlicedEllpack", "f32", (16, 0)),
+                                             ("SlicedEllpack", "bf16", (32, 1))])
+def test_autotune_times_the_shape_a_matrix_is_built_with(tnl, fmt, dtype, shape):
+    # (workgroups per CU, two rows per lane) of a short-row matrix as the header documents them
+    rp, c, v = W.laplacian_3d(20)
+    _, _, allt = tnl.autotune(rp, c, v, formats=[fmt], dtype=dtype, repetitions=2)
+    assert shape in {(t["blocks_per_cu"], t["pair_rows"]) for t in allt}

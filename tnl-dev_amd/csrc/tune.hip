@@ -15,8 +15,8 @@ struct Candidate
 {
    int format;
    int lanes;      // 0: kernel default
-   int blocksPerCu;  // 0: default
-   int pairRows;   // -1: default
+   int blocksPerCu;  // 0: not a padded format
+   int pairRows;     // -1: not a padded format
    int sliceSize;  // SlicedEllpack: 16, 32 (TNL's default), 64; 0 for other formats
    int stripes;    // CSRAdaptive: column stripes of the striped plan (0: none)
 };
@@ -31,16 +31,18 @@ std::vector< Candidate > candidatesFor( int format, bool xExceedsL2 )
          for( int l : { 2, 4, 8, 16, 32 } )
             c.push_back( { format, l, 0, -1, 0, 0 } );
          break;
+      // 16 and 32 workgroups per CU with one and two rows per lane: the shape that the construction chooses is always
+      // among them (a matrix tuned over 8 and 16 only could be slower than an untuned one)
       case TNLHIP_ELLPACK:
          for( int p : { 0, 1 } )
-            for( int b : { 8, 16 } )
+            for( int b : { 16, 32 } )
                c.push_back( { format, 0, b, p, 0, 0 } );
          break;
       case TNLHIP_SLICED_ELLPACK:
          // slice sizes outermost: a change of slice size re-lays the storage out
          for( int s : { 32, 16, 64 } )
             for( int p : { 0, 1 } )
-               for( int b : { 8, 16 } )
+               for( int b : { 16, 32 } )
                   c.push_back( { format, 0, b, p, s, 0 } );
          break;
       case TNLHIP_CSR_ADAPTIVE:
@@ -57,16 +59,19 @@ std::vector< Candidate > candidatesFor( int format, bool xExceedsL2 )
    return c;
 }
 
-// Every knob of the candidate, defaults included, so a matrix configured for one candidate
-// carries nothing over from the one timed before it.
+// Every knob that the candidates of its format differ in, so a matrix configured for one candidate carries nothing
+// over from the one timed before it.  (Rows per lane and workgroups per CU are read by the padded kernels only, whose
+// candidates all name them.)
 void configure( tnlhip_matrix A, const Candidate& c )
 {
    const bool csrGroups = c.format == TNLHIP_CSR_LIGHT || c.format == TNLHIP_CSR_HYBRID ||
                           c.format == TNLHIP_CSR_VECTOR || c.format == TNLHIP_CSR_ADAPTIVE;
    if( csrGroups )
       TNLHIP_CHECK_STATUS( tnlhip_matrix_set_param( A, "lanes_per_row", c.lanes ) );
-   TNLHIP_CHECK_STATUS( tnlhip_matrix_set_param( A, "blocks_per_cu", c.blocksPerCu > 0 ? c.blocksPerCu : 16 ) );
-   TNLHIP_CHECK_STATUS( tnlhip_matrix_set_param( A, "pair_rows", c.pairRows > 0 ? 1 : 0 ) );
+   if( c.blocksPerCu > 0 ) {
+      TNLHIP_CHECK_STATUS( tnlhip_matrix_set_param( A, "blocks_per_cu", c.blocksPerCu ) );
+      TNLHIP_CHECK_STATUS( tnlhip_matrix_set_param( A, "pair_rows", c.pairRows ) );
+   }
    if( c.format == TNLHIP_SLICED_ELLPACK )
       TNLHIP_CHECK_STATUS( tnlhip_matrix_set_param( A, "slice_size", c.sliceSize > 0 ? c.sliceSize : 32 ) );
    if( c.format == TNLHIP_CSR_ADAPTIVE )
@@ -143,8 +148,7 @@ int tnlhip_autotune_csr( int value_dtype, int32_t rows, int32_t columns, const i
             }
          }
          if( kept )
-            // leave the kept matrix configured exactly as its best candidate (format defaults
-            // restored for the knobs the candidate leaves at their default)
+            // leave the kept matrix configured exactly as its best candidate
             configure( A, Candidate{ best->format, best->lanes, best->blocks_per_cu, best->pair_rows, best->slice_size,
                                      best->column_stripes } );
          else
