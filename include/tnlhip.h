@@ -217,11 +217,15 @@ int tnlhip_matrix_get_storage( tnlhip_matrix A, double* values, int32_t* columns
  * of the vector type. */
 int tnlhip_matrix_get_diagonal( tnlhip_matrix A, void* diagonal, void* stream );
 
-/* Overrides a kernel parameter chosen at construction (FP32 / BF16 ChunkedEllpack and FP32
- * SlicedEllpack start with "xcd_remap" 1; for rows of at most 8 slots on average Ellpack and FP64 / BF16 SlicedEllpack with "pair_rows" 1, "blocks_per_cu"
- * 32 and "xcd_remap" 1, but FP64 SlicedEllpack beyond 1500000 rows with "xcd_remap" 0 and FP32 Ellpack beyond
- * 3000000 rows with "xcd_remap" 3 and "pair_rows" 0; every other
- * matrix with "xcd_remap" 0, "pair_rows" 0, "blocks_per_cu" 16): "lanes_per_row" (CSR light / hybrid /
+/* Overrides a kernel parameter chosen at construction.  Matrices start with "xcd_remap" 0,
+ * "pair_rows" 0 and "blocks_per_cu" 16, but for
+ *   FP32 / BF16 ChunkedEllpack and FP32 SlicedEllpack: "xcd_remap" 1;
+ *   rows of at most 8 slots on average, Ellpack and FP64 / BF16 SlicedEllpack: "pair_rows" 1,
+ *     "blocks_per_cu" 32, "xcd_remap" 1 (FP64 SlicedEllpack beyond 1500000 rows "xcd_remap" 0, FP32
+ *     Ellpack beyond 3000000 rows "pair_rows" 0 and "xcd_remap" 3);
+ *   longer rows, FP64 / FP32 Ellpack: "xcd_remap" 3, "blocks_per_cu" 32; FP64 SlicedEllpack:
+ *     "pair_rows" 1, "blocks_per_cu" 32; BF16 SlicedEllpack: "xcd_remap" 1.
+ * The parameters: "lanes_per_row" (CSR light / hybrid /
  * vector: a power of two in [1, 64]; once set, that many lanes share each row even when rows
  * average at most 8 stored elements, where these kernels otherwise take CSRScalar's staged
  * one-lane-per-row path); "xcd_remap" (row distribution: 0 the plain order, 1 contiguous row

@@ -151,11 +151,9 @@ tnlhip_matrix_s* buildFromSegments( int format, int dtype, int32_t rows, int32_t
       M->adaptiveHost = buildAdaptiveBlocks( rows, M->meta.offsets.data(), vsize, kWave, 256, kAdaptiveStreamBytes,
                                              kAdaptiveMaxElements );
    }
-   // ChunkedEllpack and SlicedEllpack with 4-byte values: slices / row blocks in XCD order (each
-   // XCD a contiguous eighth) keep the x they gather in that XCD's L2: at 160^3 FP32 ChunkedEllpack
-   // 45.8 -> 42.3 us, SlicedEllpack 47.5 -> 45.7 us; FP64 (twice the x) measured ChunkedEllpack
-   // 70 -> 72 us and FP32 Ellpack 49.4 -> 52.1 us, so those keep the plain order
-   if( ( format == TNLHIP_CHUNKED_ELLPACK || format == TNLHIP_SLICED_ELLPACK ) && dtype != TNLHIP_F64 )
+   // ChunkedEllpack with 4-byte vectors: slices in XCD order (each XCD a contiguous eighth) keep the x they gather in
+   // that XCD's L2: at 160^3 FP32 45.8 -> 42.3 us; FP64 (twice the x) 70 -> 72 us, so it keeps the plain order
+   if( format == TNLHIP_CHUNKED_ELLPACK && dtype != TNLHIP_F64 )
       M->xcdRemap = 1;
    // Row distribution and rows per lane of the padded formats, from a sweep of both and of 8 to 64
    // workgroups per CU over Laplacians of 100^3, 127 x 150 x 93, 160^3 and 2000^2 rows (us; each row is summed
@@ -163,33 +161,34 @@ tnlhip_matrix_s* buildFromSegments( int format, int dtype, int32_t rows, int32_t
    // workgroups per CU suit all but FP32 SlicedEllpack:
    //   SlicedEllpack FP64  one row, plain order 23.1 38.2 75.6 59.5; two rows 20.6 33.3 69.6 51.6, in XCD
    //                       order 18.7 33.9 71.7 52.9 (taken up to 1.5 million rows)
-   //   SlicedEllpack FP32  one row, XCD order, 16 per CU 13.2 21.8 46.8 36.1
+   //   SlicedEllpack FP32  one row, XCD order, 16 per CU 13.2 21.8 46.8 36.1 (y = y - A x: 13.5 22.8 50.9 40.1; two
+   //                       rows, XCD order 14.4 24.9 57.9 41.6)
    //   SlicedEllpack BF16  one row, XCD order 12.3 34.0 66.9 52.4; two rows, XCD order 12.2 20.5 44.9 32.8
    //   Ellpack FP64        one row, each XCD striding over its eighth 23.5 41.5 73.5 60.7; two rows, XCD
    //                       order 17.9 33.1 70.8 53.8
-   //   Ellpack FP32        the same 16.8 28.8 50.3 41.5 and 13.7 23.2 51.3 38.3 (taken up to 3 million rows)
+   //   Ellpack FP32        the same 16.8 28.8 50.3 41.5 and 13.7 23.2 51.3 38.3 (taken up to 3 million rows: beyond
+   //                       them it is 2 % slower on the 3D box and 8 % faster on the 2D one, and the 3D order stays)
    //   Ellpack BF16        one row, plain order 14.0 35.5 83.0 60.2; two rows, XCD order 11.4 19.4 41.5 32.6
-   // Rows of more than 8 slots on average keep the shapes they had (one row per lane; BF16 SlicedEllpack on lognormal
-   // rows of 17 entries 125 us, two rows per lane 211).
-   const bool sliced = format == TNLHIP_SLICED_ELLPACK;
+   // Rows of more than 8 slots on average keep the shapes they had before that sweep: FP64 SlicedEllpack two rows per
+   // lane in plain order (160^3 76.1 -> 73.2 us), the others one (BF16 SlicedEllpack on lognormal rows of 17 entries
+   // 125 us, two rows per lane 211).
+   const bool sliced = format == TNLHIP_SLICED_ELLPACK, ellpack = format == TNLHIP_ELLPACK;
    const bool shortRows = M->meta.allocated <= 8 * (int64_t) rows;
-   if( ! shortRows ) {
-      if( sliced && dtype != TNLHIP_F64 )
-         M->xcdRemap = 1;
-      if( format == TNLHIP_ELLPACK && dtype != TNLHIP_BF16 )
+   if( ellpack && ! shortRows ) {
+      if( dtype != TNLHIP_BF16 ) {
          M->xcdRemap = 3;
-      if( ( format == TNLHIP_ELLPACK && dtype != TNLHIP_BF16 ) || ( sliced && dtype == TNLHIP_F64 ) )
          M->blocksPerCu = 32;
-      if( sliced && dtype == TNLHIP_F64 )
-         M->pairRows = 1;
+      }
    }
-   else if( ( sliced && dtype != TNLHIP_F32 ) || format == TNLHIP_ELLPACK ) {
+   else if( sliced && ( dtype == TNLHIP_F32 || ( ! shortRows && dtype != TNLHIP_F64 ) ) )
+      M->xcdRemap = 1;
+   else if( sliced || ellpack ) {
       M->blocksPerCu = 32;
       M->pairRows = 1;
       M->xcdRemap = 1;
-      if( sliced && dtype == TNLHIP_F64 && rows > 1500000 )
+      if( sliced && dtype == TNLHIP_F64 && ( ! shortRows || rows > 1500000 ) )
          M->xcdRemap = 0;
-      if( format == TNLHIP_ELLPACK && dtype == TNLHIP_F32 && rows > 3000000 ) {
+      if( ellpack && dtype == TNLHIP_F32 && rows > 3000000 ) {
          M->pairRows = 0;
          M->xcdRemap = 3;
       }
