@@ -4,10 +4,12 @@
 // caller with k of them (block Krylov methods, many time levels, the solve server's requests)
 // would read the matrix k times.  Here the matrix is read once: X and Y are row-major (entry
 // row * k + j), a row is taken by KP / VW lanes (KP = k rounded up to a power of two), each lane
-// keeping VW adjacent right-hand sides as one 16-byte load and store (two FP64 or four FP32
-// columns when k is a multiple of VW and X, Y are 16-byte aligned; VW = 1 otherwise); the lanes
-// of a row load the same stored element (one transaction) while their gathers of x at that column
-// are contiguous, and each lane keeps 8 slots' loads in flight.  Each column is summed left to right
+// keeping VW adjacent right-hand sides.  multiProductKernel: VW is two FP64 or four FP32 columns, one
+// 16-byte load and store, when k is a multiple of it and X, Y are 16-byte aligned, and 1 otherwise; the
+// lanes of a row load the same stored element (one transaction) while their gathers of x at that column
+// are contiguous, and each lane keeps 8 slots' loads in flight.  multiShortKernel, for matrices whose
+// every row has at most 8 slots: several columns a lane whatever k and the alignment, slots shared through
+// LDS, the next rows' loads under way (launchShort's rule).  Each column is summed left to right
 // over the row's slots, rounding each product (TNL's Host order: CSRScalarKernel.hpp:70-107 and
 // the padded formats' per-segment loops), so column j of Y equals TNL's product of column j of X
 // bit for bit; padding slots (column -1) are skipped.  Keepers as SparseMatrixView.hpp:447-471.
@@ -69,9 +71,9 @@ __device__ __forceinline__ A lane( const T& v, int i )
 
 // A row is taken by L = KP / VW lanes; lane jq holds columns VW jq .. VW jq + VW - 1 of X and Y,
 // loaded and stored VW at a time (VW > 1 only when k % VW == 0 and X, Y are 16-byte aligned).
-// Workgroup b works on logical row block (b % 8) * (grid / 8) + b / 8, so each XCD takes a
-// contiguous eighth of the rows and the x rows a block gathers stay in that XCD's L2 (the grid is
-// a multiple of 8; blocks past the last row exit).
+// Workgroup b works on logical row block multiBlock( chunk ): the rows go to the XCDs in shares of `chunk`
+// blocks, so that the x rows a block gathers stay in its XCD's L2 (the grid is a multiple of 8 shares;
+// blocks past the last row exit).
 template< int KP, int VW, typename V, typename A, typename Y, typename View >
 __global__ __launch_bounds__( 256 ) void multiProductKernel( View view, const int32_t* __restrict__ col,
                                                              const V* __restrict__ val, int32_t k,

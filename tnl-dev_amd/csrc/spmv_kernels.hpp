@@ -436,12 +436,12 @@ __global__ __launch_bounds__( 256 ) void csrAdaptiveKernel( int32_t nblocks, con
 
 // ------------------------------------------------------------------ Ellpack / SlicedEllpack
 
-// One lane per row, column-major storage: consecutive lanes read consecutive addresses
-// for every local index (EllpackView.hpp:361-378, SlicedEllpackView.hpp:248-290).  The
-// slots of a row are read eight at a time with unconditional loads (indexes past the row
-// end are clamped to its last slot, padding gathers x[0]), so 24 loads per lane are in
-// flight; the sum still runs left to right over the non-padding slots only, which is the
-// Host result bit for bit.  Each workgroup owns `rowsPerBlock` consecutive rows.
+// One or two adjacent rows per lane, column-major storage: consecutive lanes read consecutive
+// addresses for every local index (EllpackView.hpp:361-378, SlicedEllpackView.hpp:248-290).  The
+// slots of a row are read eight at a time, their loads in flight together (24 with the gathers of
+// x); the sum still runs left to right over the non-padding slots only, which is the Host result
+// bit for bit.  What becomes of a chunk's slots beyond the row's end: paddedRows.  Each workgroup
+// owns `rowsPerBlock` consecutive rows.
 constexpr int kChunk = 8;
 constexpr int kRowsInFlight = 2;  // rows per lane per iteration of the padded kernels
 
