@@ -236,6 +236,97 @@ def test_fused_iterations_follow_the_oracle(tnl, dev, fmt, n):
             np.testing.assert_allclose(xd.cpu().numpy(), ref["x"], rtol=0, atol=1e-8 * np.abs(ref["x"]).max())
 
 
+def _follow(tnl, dev, rp, cols, vals, fmt, dt, steps, method, pre, rtol):
+    """The first residuals of a solve follow the oracle's; x at an odd element offset."""
+    b = W.uniform_vector(len(rp) - 1, 11)
+    p = dict(convergence_residue=1e-30, max_iterations=steps, preconditioner=pre)
+    ref = O.solve(method, rp, cols, vals, b, **p)
+    A = tnl.SparseMatrix.from_csr(rp, cols, vals, format=fmt, dtype=dt)
+    s = tnl.getLinearSolver(method)
+    s.setMatrix(A)
+    s.setup(**p)
+    x = torch.zeros(len(b) + 1, dtype=A.vector_dtype, device=dev)[1:]
+    s.solve(t(b, dev, A.vector_dtype), x)
+    h = s.getResidualHistory()
+    assert len(h) >= steps and s.getIterations() == ref["iterations"]
+    np.testing.assert_allclose(h[:steps], ref["history"][:steps], rtol=rtol)
+    np.testing.assert_allclose(x.cpu().numpy(), ref["x"], rtol=0, atol=rtol * np.abs(ref["x"]).max())
+
+
+@pytest.mark.parametrize("method", ["cg", "bicgstab"])
+@pytest.mark.parametrize("fmt,dt,n", [("CSRScalar", "f64", 299999), ("CSRScalar", "f64", 600001), ("CSRScalar", "f32", 299999),
+                                      ("SlicedEllpack", "f64", 600001), ("SlicedEllpack", "f32", 70001),
+                                      ("SlicedEllpack", "f32", 600001), ("Ellpack", "f32", 300001),
+                                      ("ChunkedEllpack", "f32", 70001)])
+def test_large_and_single_precision_fused_solves_follow_the_oracle(tnl, dev, method, fmt, dt, n):
+    # 299999 CSR rows: 1172 partials, more than a fold loads ahead, with the operand formed in the product; beyond 300000
+    # rows the direction has a pass of its own; FP32: four-wide lanes with one, two or three entries left over
+    i = np.arange(n)
+    r, c = np.concatenate([i[1:], i, i[:-1]]), np.concatenate([i[1:] - 1, i, i[:-1] + 1])
+    up = -1.0 if method == "cg" else -0.7
+    v = np.concatenate([np.full(n - 1, -1.0), 2.6 + 0.3 * np.cos(i), np.full(n - 1, up)])
+    o = np.lexsort((c, r))
+    rp = np.zeros(n + 1, np.int32)
+    np.cumsum(np.bincount(r, minlength=n), out=rp[1:])
+    for pre in (0, 1):
+        # FP64: sums of 600001 products in another order, 1e-13 each, amplified by the steps; FP32: six steps that round
+        # vectors of a system of condition 5 at 6e-8
+        _follow(tnl, dev, rp, c[o].astype(np.int32), v[o], fmt, dt, 10 if dt == "f64" else 6, method, pre,
+                1e-8 if dt == "f64" else 1e-4)
+
+
+@pytest.mark.parametrize("method", ["cg", "bicgstab"])
+@pytest.mark.parametrize("fmt", ["CSRAdaptive", "CSRVector", "CSRLight", "Ellpack", "SlicedEllpack", "ChunkedEllpack", "BiEllpack"])
+@pytest.mark.parametrize("dt", ["f64", "f32"])
+def test_fused_solves_of_long_rows_follow_the_oracle(tnl, dev, method, fmt, dt):
+    # 30 entries a row on average, some rows of 700 (a wavefront's in CSRAdaptive) and of 2600 (a workgroup's)
+    n = 4099
+    rng = np.random.default_rng(7)
+    L = np.full(n, 14)
+    L[[5, 900, 4000]] = 700
+    L[[77, 78, 2500]] = 2600
+    r = np.repeat(np.arange(n), L)
+    c = np.concatenate([rng.choice(n, k, replace=False) for k in L])
+    w = rng.uniform(-1, 1, len(r))
+    key, first = np.unique(np.concatenate([r * n + c, c * n + r]), return_index=True)
+    v = np.concatenate([w, w])[first]
+    r, c = key // n, key % n
+    v[r == c] = 0.0
+    v[(r == c)] = 1.0 + np.bincount(r, weights=np.abs(v), minlength=n)[r[r == c]]
+    if method == "cg":  # one value for both halves
+        v = np.where(r > c, 0.0, v)
+        low = np.searchsorted(key, c * n + r)
+        v = np.where(r > c, v[low], v)
+        v[r == c] = 1.0 + np.bincount(r[r != c], weights=np.abs(v[r != c]), minlength=n)[r[r == c]]
+    missing = np.setdiff1d(np.arange(n), r[r == c])  # rows without a diagonal entry get one
+    extra = 1.0 + np.bincount(r[r != c], weights=np.abs(v[r != c]), minlength=n)[missing]
+    r, c, v = np.concatenate([r, missing]), np.concatenate([c, missing]), np.concatenate([v, extra])
+    o = np.lexsort((c, r))
+    rp = np.zeros(n + 1, np.int32)
+    np.cumsum(np.bincount(r, minlength=n), out=rp[1:])
+    for pre in (0, 1):
+        # FP32: rows of 34 products on average round at 34 * 6e-8 of the residual before, up to 20 times the new one, four
+        # times over
+        _follow(tnl, dev, rp, c[o].astype(np.int32), v[o], fmt, dt, 6 if dt == "f64" else 4, method, pre,
+                1e-8 if dt == "f64" else 5e-4)
+
+
+@pytest.mark.parametrize("method,n", [("cg", 100000), ("cg", 100001), ("bicgstab", 100001)])
+def test_rows_of_64_lanes_on_both_sides_of_the_fused_limit(tnl, dev, method, n):
+    i = np.arange(n)
+    d = [k for k in range(-6, 7)]
+    r = np.concatenate([i[max(0, -k):n - max(0, k)] for k in d])
+    c = np.concatenate([i[max(0, -k):n - max(0, k)] + k for k in d])
+    v = np.where(r == c, 14.0, -1.0 / (1 + np.abs(r - c)))
+    if method == "bicgstab":
+        v = np.where(c > r, 0.7 * v, v)
+    o = np.lexsort((c, r))
+    rp = np.zeros(n + 1, np.int32)
+    np.cumsum(np.bincount(r, minlength=n), out=rp[1:])
+    # (four steps: the residual falls 150 times a step)
+    _follow(tnl, dev, rp, c[o].astype(np.int32), v[o], "CSRVector", "f64", 4, method, 1, 1e-8)
+
+
 def _arrow(n, m):
     """Tridiagonal with m more entries in row 0 and column 0, symmetric and diagonally dominant."""
     i = np.arange(n)
