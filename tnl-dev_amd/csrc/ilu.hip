@@ -19,9 +19,9 @@
 // The triangular solves work on a copy of the factor in level order (Sweep): the rows of a level,
 // longest first, take consecutive positions from an even one on, and vectors are permuted to
 // positions before the first level and back after the last one.  A level with more than
-// kNarrowLevel rows is one launch over the device; runs of consecutive smaller levels are one
-// launch of a single 1024-lane workgroup, which takes up to kStepRows rows at a time (a step), two
-// adjacent positions per lane.
+// kNarrowLevel rows, or more than kFarLevel of them that reach far back, is one launch over the
+// device; runs of consecutive smaller levels are one launch of a single workgroup, as large as the
+// largest of them needs (up to 1024 lanes), which takes two adjacent positions per lane at a time (a step).
 //
 // 64^3 7-point convection-diffusion in FP64 (190 levels a sweep): BiCGStab to 1e-10, 58 iterations.
 // One launch per level above 1024 rows and a workgroup for the others, each row reading its row
@@ -38,7 +38,6 @@ namespace {
 
 constexpr int kIluBlock = 256;
 constexpr int kRunBlock = 1024;         // one workgroup of 16 waves for runs of small levels
-constexpr int32_t kStepRows = 2 * kRunBlock;
 constexpr int32_t kSliceRows = 2 * kWave;
 constexpr int32_t kNarrowLevel = 4096;  // levels of at most this many rows are taken in runs
 constexpr int32_t kFarLevel = 1024;     // and these where some entry is older than the ring
@@ -412,7 +411,9 @@ __global__ __launch_bounds__( kRunBlock ) void sweepRunKernel( SweepView< T > f,
 }
 
 // Entries of a row fetched ahead (W), and how many steps ahead (D): 3 entries cover the lower and the
-// upper half of a 7-point stencil; D is what the 128 registers of a lane hold.
+// upper half of a 7-point stencil; D is what the 128 registers of a lane hold.  Factors of more than 3
+// entries a row take 7 two steps ahead (ms per iteration of BiCGStab, 3 four ahead / 7 two ahead: 9-point
+// 300^2 9.2 / 3.0, 27-point 60^3 10.8 / 8.2, 120^3 54.6 / 36.3).
 constexpr int kShortW = 3, kShortD = 4, kLongW = 7, kLongD = 2;
 
 // Rows grouped by level, in a level the rows with the most entries first (`length`, without U's
