@@ -52,12 +52,7 @@ Workspace& threadWorkspace()
 void Matrix::uploadMetadata()
 {
    switch( meta.kind ) {
-      case KIND_CSR:
-         offsets.upload( meta.offsets );
-         waveMost = 0;
-         for( int32_t r = 0; r < rows; r += kWave )
-            waveMost = std::max( waveMost, meta.offsets[ std::min( r + kWave, rows ) ] - meta.offsets[ r ] );
-         break;
+      case KIND_CSR: offsets.upload( meta.offsets ); break;
       case KIND_SLICED:
          sliceOffsets.upload( meta.sliceOffsets );
          sliceSizes.upload( meta.sliceSegmentSizes );

@@ -47,6 +47,7 @@ struct HostSegments
    int64_t storage = 0;    // getStorageSize()
    int64_t allocated = 0;  // elements that can hold data
    int32_t rowMost = 0;    // most slots of a row (CSR, Ellpack, SlicedEllpack)
+   int32_t waveMost = 0;   // CSR: most slots of 64 consecutive rows (from a multiple of 64 on)
    // CSR
    std::vector< int32_t > offsets;
    // Ellpack
@@ -108,7 +109,6 @@ struct Matrix
    int32_t lanes = 0;      // lanes per row for CSR light / hybrid / vector
    int32_t defaultLanes = 0;  // the format's own choice, restored by lanes_per_row 0
    bool lanesExplicit = false;  // lanes_per_row set by the caller: the cooperative kernel always runs
-   int32_t waveMost = 0;  // CSR: most stored elements in 64 consecutive rows (from a multiple of 64 on)
    int32_t reach = 0;  // max |column - row| over the stored entries when the storage was filled (a hint; 0: unknown)
    int32_t xcdRemap = 0;
    // every chunk of a ChunkedEllpack matrix keeps its padding after its elements (true for

@@ -21,12 +21,21 @@ inline int32_t ceilDiv( int32_t a, int32_t b ) { return a / b + ( a % b != 0 ); 
 void csrOffsets( HostSegments& s, const int32_t* caps )
 {
    s.offsets.resize( (size_t) s.n + 1 );
-   int64_t run = 0;
-   for( int32_t i = 0; i < s.n; i++ ) {
-      s.offsets[ i ] = (int32_t) run;
-      run += caps[ i ];
-      s.rowMost = std::max( s.rowMost, caps[ i ] );
+   int64_t run = 0, waveMost = 0;
+   int32_t most = 0;
+   int32_t* offsets = s.offsets.data();
+   for( int64_t b = 0; b < s.n; b += 64 ) {  // a wavefront's rows
+      const int64_t begin = run, end = std::min< int64_t >( b + 64, s.n );
+      for( int64_t i = b; i < end; i++ )  // (apart from the prefix sum, whose chain it would lengthen)
+         most = std::max( most, caps[ i ] );
+      for( int64_t i = b; i < end; i++ ) {
+         offsets[ i ] = (int32_t) run;
+         run += caps[ i ];
+      }
+      waveMost = std::max( waveMost, run - begin );
    }
+   s.rowMost = most;
+   s.waveMost = (int32_t) std::min< int64_t >( waveMost, std::numeric_limits< int32_t >::max() );
    if( run > std::numeric_limits< int32_t >::max() )
       throw Error( TNLHIP_ERROR_CAPACITY, "CSR storage exceeds the int32 index range" );
    s.offsets[ s.n ] = (int32_t) run;

@@ -939,7 +939,7 @@ template< typename A >
 bool stagedThroughout( const Matrix& M )
 {
    return kindOf( M.format ) == KIND_CSR && lanesPerRow( M ) == 0 && M.meta.allocated <= (int64_t) kShortRow * M.rows &&
-          M.waveMost <= kAdaptiveStreamBytesPerWave / (int) sizeof( A );
+          M.meta.waveMost <= kAdaptiveStreamBytesPerWave / (int) sizeof( A );
 }
 
 // Launches the row kernel of M's format over rows [first, last) and returns its grid, or with `dry`
