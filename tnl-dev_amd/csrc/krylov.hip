@@ -19,6 +19,12 @@ struct FusedKeeper
    ReduceSlot out;
    Gate gate;
    double acc[ Op::kSums ] = {};
+   __device__ __forceinline__ bool shut() const
+   {
+      if constexpr( Op::kStored )
+         return Op::shut( gate );
+      return false;
+   }
    __device__ __forceinline__ void prefetch() { op.prefetch( gate ); }
    __device__ __forceinline__ bool begin() { return op.begin(); }
    __device__ __forceinline__ Y at( const Y* x, int64_t c ) const { return op.at( x, c ); }

@@ -11,11 +11,12 @@
 // order and round each product and sum separately, so they reproduce the Host result bit
 // for bit; the cooperative kernels reassociate the row sum.
 //
-// A kernel asks its keeper for everything beside the matrix: closed() (a plain product's gate),
-// prefetch() and begin() (called by every thread before the first at(); begin: false, for the whole
-// grid alike, when there is nothing to do), at( x, c ) (entry c of the operand), keep( row, sum )
-// (once per row, by one lane) and finish() (called by every thread after the rows).  The kernels of
-// short rows call begin() behind the loads of their first elements, which do not depend on it.
+// A kernel asks its keeper for everything beside the matrix: closed() (a plain product's gate), shut()
+// (the gate of a fused product that has nothing to fold; the same for the whole grid), prefetch() and
+// begin() (called by every thread before the first at(); begin: false, for the whole grid alike but for
+// a gate that is being closed, when there is nothing to do), at( x, c ) (entry c of the operand),
+// keep( row, sum ) (once per row, by one lane) and finish() (called by every thread after the rows).  The
+// kernels of short rows call begin() behind the loads of their first elements, which do not depend on it.
 #pragma once
 
 #include "spmv.hpp"
@@ -42,8 +43,10 @@ __device__ __forceinline__ bool openKeeper( Keep& keep )
    if constexpr( Keep::kPlain )
       return ! keep.closed();
    else {
+      if( keep.shut() )
+         return false;
       keep.prefetch();
-      return __syncthreads_and( keep.begin() );
+      return Keep::kStored || __syncthreads_and( keep.begin() );
    }
 }
 
@@ -296,8 +299,11 @@ __global__ __launch_bounds__( 256 ) void csrScalarStagedKernel( const int32_t* _
       if( keep.closed() )
          return;
    }
-   else
+   else {
+      if( keep.shut() )
+         return;
       keep.prefetch();
+   }
    csrScalarStagedRows< K, V, A, Y, Keep >( off, col, val, x, keep, first, last, remap );
    keep.finish();
 }
@@ -691,8 +697,11 @@ __global__ __launch_bounds__( 256 ) void ellpackKernel( EllpackSlots slots, cons
                                                         Keep keep, int32_t first, int32_t last,
                                                         int32_t rowsPerBlock, int dist )
 {
-   if constexpr( PAIR && ! Keep::kPlain )
+   if constexpr( PAIR && ! Keep::kPlain ) {
+      if( keep.shut() )
+         return;
       keep.prefetch();  // begin() follows the first loads
+   }
    else if( ! openKeeper( keep ) )
       return;
    const int64_t base = PAIR ? ( first & ~1 ) : first;
@@ -706,8 +715,11 @@ __global__ __launch_bounds__( 256 ) void slicedKernel( SlicedSlots slots, const 
                                                        Keep keep, int32_t first, int32_t last,
                                                        int32_t rowsPerBlock, int dist )
 {
-   if constexpr( PAIR && ! Keep::kPlain )
+   if constexpr( PAIR && ! Keep::kPlain ) {
+      if( keep.shut() )
+         return;
       keep.prefetch();  // begin() follows the first loads
+   }
    else if( ! openKeeper( keep ) )
       return;
    const int64_t base = PAIR ? ( first & ~1 ) : first;
