@@ -495,13 +495,13 @@ def test_launches_behind_the_stop_leave_the_matrix_alone(tnl, dev):
     took = {}
     for most in (10, 13):
         s.setup(convergence_residue=1e-300, max_iterations=most)
-        for _ in range(8):
+        for _ in range(12):
             x = torch.zeros_like(b)
             torch.cuda.synchronize()
             start = time.perf_counter()
             s.solve(b, x)
             took[most] = min(took.get(most, 1e9), time.perf_counter() - start)
-    assert took[13] < 1.66 * took[10], took
+    assert took[13] < 1.7 * took[10], took
 
 
 @pytest.mark.parametrize("method,vectors", [("cg", 4), ("bicgstab", 7)])
